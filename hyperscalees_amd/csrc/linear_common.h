@@ -157,8 +157,9 @@ struct LifOut {
 };
 
 int launch_linear_small(LinParams& P, DeviceState* st, hipStream_t s);
-// fp32 math, do_mm, rank <= 16: the members' A_m / B_m rows into the workspace,
-// then an fp32 MFMA GEMM with x B_m and (x B_m) A_m^T fused (linear_f32.hip).
+// fp32 math, rank <= 16: the members' A_m / B_m rows and W's bf16 parts into the
+// workspace, then an MFMA GEMM on split operands with x B_m and (x B_m) A_m^T
+// fused (linear_f32.hip).
 int launch_linear_f32(LinParams& P, DeviceState* st, hipStream_t s, void* work, size_t work_bytes);
 // Every member's (a + b) x r factor rows into F (n (a + b) r floats), the
 // scaled role's rows (do_mm: A; do_Tmm: the input side) times sign * sigma / sqrt(r).

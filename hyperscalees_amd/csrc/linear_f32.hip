@@ -5,16 +5,31 @@
 //
 // Two launches:
 //   k_factors   every member's B_m (stream rows [0, b)) and scaled A_m (rows
-//             [b, a + b)) into the workspace, each row drawn once.
+//             [b, a + b)) into the workspace, each row drawn once; for
+//             k_gemm_f32s its last blocks split W into three bf16 parts.
 //   k_gemm_f32  y = x W^T with fp32 MFMA (32x32x2) over 128-row x BN-column
 //             tiles, K in chunks of 32 staged through double-buffered LDS with
 //             the chunk's B_m rows beside them; each thread also accumulates
 //             x B_m for its row on the vector ALU from the staged chunk, and the
 //             epilogue adds (x B_m) A_m^T with the tile's A_m rows.
-// The LDS copy of a chunk stores each row's 32 k values as the even k then the
-// odd k, so a lane (row l % 32, k-group l / 32 of the 32x32x2 MFMA) reads its
-// 16 k-steps of a chunk with four 16-byte loads.
+//   k_gemm_f32s  the same product on bf16 MFMA (32x32x16) with split operands.
+//             An fp32 value is the exact sum of three bf16 parts of 8 significant
+//             bits, x = x0 + x1 + x2, so x w needs the six products x0 w0, x0 w1,
+//             x1 w0, x1 w1, x0 w2, x2 w0 (the others are below 2^-25 |x w|); bf16
+//             activations and spikes are one part: three products.  Products of
+//             two parts are exact in the fp32 accumulator.  Six bf16 MFMAs take
+//             3/8 of the matrix-core time of the eight fp32 MFMAs they replace:
+//             65536 x 1024 -> 1024 at rank 1 (16 rows per member) 1638 -> 855 us,
+//             161 TFLOP/s of fp32 product and 964 of issued bf16, against 1144 of a
+//             large bf16 product on the same card; error against float64 5.3e-7
+//             -> 2.7e-7 (a step of 16 k rounds the leading sum once, not eight
+//             times).  Which of the two runs: f32_split_shape.
+// The LDS copy of a chunk of k_gemm_f32 stores each row's 32 k values as the
+// even k then the odd k, so a lane (row l % 32, k-group l / 32 of the 32x32x2
+// MFMA) reads its 16 k-steps of a chunk with four 16-byte loads.
 #include <math.h>
+
+#include <type_traits>
 
 #include "linear_common.h"
 #include "noise_dev.h"
@@ -23,11 +38,13 @@
 namespace hses {
 
 constexpr int KF_BM = 128, KF_BK = 32, KF_THREADS = 256;
-constexpr int KF_XP = 36;          // LDS pitch of a staged row (floats): 16 even k, 16 odd k, pad
+constexpr int KF_XP = 36;          // k_gemm_f32: LDS pitch of a staged row (floats): 16 even k, 16 odd k, pad
 constexpr int KF_AMAX = 8192;      // floats of A rows a workgroup keeps for its epilogue
 constexpr int KF_RMAX = 16;        // ranks handled
+constexpr int KS_BPT = 2;          // k_gemm_f32s: B_m chunk values staged per thread
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x16 mfma32x2(float a, float b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
@@ -46,14 +63,65 @@ __device__ __forceinline__ float x_at(const void* x, int64_t off, int32_t k) {
     }
 }
 
+// The three bf16 parts of v: v = p[0] + p[1] + p[2] exactly for normal v (8 + 8
+// + 8 significant bits, each part rounded to nearest), as pairs of consecutive k.
+__device__ __forceinline__ void split3(float lo, float hi, uint32_t (&p)[3]) {
+    p[0] = pack_bf16x2(lo, hi);
+    const float l1 = lo - __uint_as_float(p[0] << 16), h1 = hi - __uint_as_float(p[0] & 0xffff0000u);
+    p[1] = pack_bf16x2(l1, h1);
+    p[2] = pack_bf16x2(l1 - __uint_as_float(p[1] << 16), h1 - __uint_as_float(p[1] & 0xffff0000u));
+}
+
+// Slot of 16-byte piece s (8 k) of row `row` in its 64-byte LDS row: a lane of
+// a quarter-wave reads the same piece of eight consecutive rows, which the XOR
+// puts on distinct banks.
+__device__ __forceinline__ int slot_of(int row, int s) { return s ^ ((row >> 1) & 3); }
+
+// Item i of the split of W: a piece of 8 k of one output row.
+__device__ __forceinline__ void split_w(const LinParams& P, uint16_t* Wp, int32_t a_pad, int64_t i) {
+    const int32_t nch = (P.b + KF_BK - 1) / KF_BK;
+    if (i >= (int64_t)nch * a_pad * 4) return;
+    // consecutive lanes: the pieces of a row (W rows contiguous in k), or for
+    // do_Tmm the output rows (W columns contiguous in the output)
+    const int32_t ch = (int32_t)(i / (a_pad * 4)), e = (int32_t)(i - (int64_t)ch * a_pad * 4);
+    const int32_t o = P.tmm ? e % a_pad : e >> 2, pc = P.tmm ? e / a_pad : e & 3;
+    const int32_t k0 = ch * KF_BK + 8 * pc;
+    const int64_t w0 = P.tmm ? (int64_t)k0 * P.a + o : (int64_t)o * P.b + k0;
+    const int64_t wk = P.tmm ? P.a : 1;
+    uint32_t d[3][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const bool ok = o < P.a;
+        const float lo = ok && k0 + 2 * u < P.b ? P.W[w0 + 2 * u * wk] : 0.0f;
+        const float hi = ok && k0 + 2 * u + 1 < P.b ? P.W[w0 + (2 * u + 1) * wk] : 0.0f;
+        uint32_t p[3];
+        split3(lo, hi, p);
+#pragma unroll
+        for (int w = 0; w < 3; ++w) d[w][u] = p[w];
+    }
+#pragma unroll
+    for (int w = 0; w < 3; ++w)
+        reinterpret_cast<uint4*>(Wp)[((int64_t)(ch * 3 + w) * a_pad + o) * 4 + slot_of(o, pc)] =
+            uint4{d[w][0], d[w][1], d[w][2], d[w][3]};
+}
+
 // ---- k_factors -------------------------------------------------------------------
 // F[m] = the member's (a + b) x r stream rows as drawn, except that the
 // rows carrying sign * sigma / sqrt(r) are scaled: do_mm's A rows [b, a + b),
 // do_Tmm's input-side rows [a, a + b) (with a the output width).  A thread
 // draws rows [q rc, q rc + rc) of one member after one jump to the group's start.
+// Blocks from fblocks on split W for k_gemm_f32 (Wp, NULL without one): with
+// a_pad output rows, [k chunk of 32][part][output row][32], the 16-byte pieces
+// of a row swizzled as k_gemm_f32 reads them from LDS (slot_of), zero past a
+// and b.  A block takes 256 pieces of 8 k.
 __global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_t groups,
-                                                 float* __restrict__ F) {
+                                                 float* __restrict__ F, int32_t fblocks,
+                                                 uint16_t* __restrict__ Wp, int32_t a_pad) {
     __shared__ BmTables t;
+    if ((int32_t)blockIdx.x >= fblocks) {
+        split_w(P, Wp, a_pad, (int64_t)(blockIdx.x - fblocks) * 256 + threadIdx.x);
+        return;
+    }
     load_bm_tables(&t, P.tables);
     __syncthreads();
     const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -69,6 +137,319 @@ __global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_
     const int32_t split = ((P.tmm ? P.a : P.b) - row0) * r;  // normals before the first scaled row
     bm_run(s, min(rc, rows - row0) * r, ctx,
            [&](int32_t i, float v) { dst[i] = i >= split ? v * sc : v; });
+}
+
+// ---- k_gemm_f32s -----------------------------------------------------------------
+__device__ __forceinline__ f32x16 mfma_bf(const u16x8& a, const u16x8& b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// What bounds it: the matrix cores.  The x chunk goes global -> registers (one
+// chunk ahead) -> three parts in LDS, W arrives split (its conversion would
+// repeat in every row tile); 48 KB of LDS and two waves per SIMD let two
+// workgroups share a CU, one's conversion and barriers beside the other's MFMAs.
+// A BM x BN tile, four waves: 2 x 2 of (BM / 2) x 64 for BN = 128, 2 x 2 of 32 x 32
+// for 64 x 64, else four of 32 rows.  RK is the rank padded to 1, 4, 8 or 16
+// (the LDS copies of B_m and A_m rows hold RK values per row, zero past r).
+template <int XFMT, int BM, int BN, int RK>
+__global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+void k_gemm_f32s(LinParams P, const float* __restrict__ F, const uint16_t* __restrict__ Wp, int32_t a_pad,
+                 int32_t bch) {
+    constexpr bool SQ = BN == 128 || BM == 64;          // 2 x 2 waves
+    constexpr int WM = SQ ? BM / 2 : 32, WN = SQ ? BN / 2 : BN;
+    constexpr int MI = WM / 32, NJ = WN / 32;           // 32 x 32 MFMA tiles of a wave
+    constexpr int NP = XFMT == HSES_FMT_F32 ? 3 : 1;    // parts of x
+    constexpr bool XLDS = XFMT != HSES_FMT_BITS;        // bits are expanded from registers
+    constexpr int TPR = KF_THREADS / BM, KPT = KF_BK / TPR;  // threads per x row, k per thread
+    extern __shared__ __align__(16) unsigned char smem[];
+    // x parts [NP][BM][32], W parts [3][BN][32] (bf16, 64-byte rows, pieces
+    // swizzled by slot_of), the chunk's B_m rows [lm][32][RK], the tile's A_m
+    // rows [lm][BN][RK], then per row the y and x offsets and the member.
+    uint16_t* Xs = reinterpret_cast<uint16_t*>(smem);
+    uint16_t* Ws = Xs + (XLDS ? NP * BM * KF_BK : 0);
+    float* Bc = reinterpret_cast<float*>(Ws + 3 * BN * KF_BK);
+    int64_t* yoffs = reinterpret_cast<int64_t*>(Bc + bch);
+    int64_t* xoffs = yoffs + BM;
+    int32_t* rlm = reinterpret_cast<int32_t*>(xoffs + BM);
+    float* As = reinterpret_cast<float*>(rlm + BM);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int32_t lc = lane & 31, kh = lane >> 5;
+    const int wm0 = SQ ? (wave >> 1) * WM : wave * 32, wn0 = SQ ? (wave & 1) * WN : 0;
+    // Tile of this workgroup: workgroups are dealt to the 8 XCDs in turn, so
+    // XCD x gets the contiguous tile range x * nb / 8 .. with the column tiles
+    // of a row tile adjacent: the workgroups that read the same x rows run on
+    // one XCD together and share its L2.
+    int64_t L0;
+    int32_t o0;
+    {
+        const uint32_t nb = gridDim.x, g = blockIdx.x, xcd = g & 7u, j = g >> 3;
+        const uint32_t q = nb >> 3, rem = nb & 7u;
+        const uint32_t ncol = (uint32_t)((P.a + BN - 1) / BN);
+        const uint32_t t = ncol == 1 ? g  // one column tile: no x rows are shared
+                           : xcd < rem ? xcd * (q + 1) + j : rem * (q + 1) + (xcd - rem) * q + j;
+        L0 = (int64_t)(t / ncol) * BM;
+        o0 = (int32_t)(t % ncol) * BN;
+    }
+    const int32_t ct = min(BN, P.a - o0);
+    const int32_t r = P.r, b = P.b;
+    const int32_t rows_here = (int32_t)min<int64_t>(BM, P.total - L0);
+    const TileRows tr(P, L0);
+    const int32_t nm = tr.member(P, rows_here - 1) + 1;
+    const bool noisy = r > 0;
+    const int64_t fpitch = (int64_t)(P.a + b) * r;  // floats of one member's factors
+    const float* Fm = F + (int64_t)tr.m_first * fpitch;
+    const int32_t in_off = P.tmm ? P.a : 0, out_off = P.tmm ? 0 : b;  // factor rows by role
+
+    if (tid < BM) {
+        const bool ok = tid < rows_here;
+        yoffs[tid] = ok ? tr.offset(P, tid, P.y_stride, P.y_plane) + o0 : 0;
+        xoffs[tid] = ok ? tr.offset(P, tid, P.x_stride, P.x_plane) : 0;
+        rlm[tid] = ok ? tr.member(P, tid) : 0;
+    }
+    // ---- the output-side factor rows of the tile's members -----------------------
+    if (noisy) {
+        for (int32_t i = tid; i < nm * BN * RK; i += KF_THREADS) {
+            const int32_t c = i % RK, o = (i / RK) % BN, lm = i / (RK * BN);
+            As[i] = (c < r && o < ct) ? Fm[lm * fpitch + (int64_t)(out_off + o0 + o) * r + c] : 0.0f;
+        }
+    }
+    __syncthreads();
+
+    // ---- staging: thread -> x row tid / TPR (KPT k), BN * 3 / 64 pieces of W ---------
+    const int xr = tid / TPR, xk = (tid % TPR) * KPT;
+    const bool xvalid = xr < rows_here;
+    const int64_t xoff = xoffs[xr];
+    const int32_t xlm = rlm[xr];
+    const bool xal = (reinterpret_cast<uintptr_t>(P.x) & 15) == 0 &&
+                     (xoff & (XFMT == HSES_FMT_F32 ? 3 : 7)) == 0;  // 16-byte loads
+    constexpr int WPC = (BN * 12 + KF_THREADS - 1) / KF_THREADS;  // 16-byte pieces per thread
+    constexpr int BPT = KS_BPT;  // B_m chunk values per thread
+    float xv[KPT];
+    u32x4 wv[WPC];
+    uint32_t xw[MI], xbits = 0;  // bit-packed x: the chunk of the MFMA rows, of row xr
+    float bv[BPT];
+    int64_t xwo[MI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) xwo[i] = XLDS ? 0 : 2 * xoffs[wm0 + 32 * i + lc];
+    // B_m chunk value j: [lm][kk][c], its float offset from Fm at chunk 0
+    int32_t boff[BPT], bkk[BPT];
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+        const int32_t e = tid + KF_THREADS * j;
+        const int32_t c = e % RK, kk = (e / RK) % KF_BK, lm = e / (RK * KF_BK);
+        bkk[j] = (e < bch && lm < nm && c < r) ? kk : b;  // b: never valid
+        boff[j] = (int32_t)(lm * fpitch) + (in_off + kk) * r + c;
+    }
+    auto b_ok = [&](int j, int32_t kc) { return kc * KF_BK + bkk[j] < b; };
+    auto load_chunk = [&](int32_t kc) {
+        const int32_t k = kc * KF_BK + xk;
+        if constexpr (!XLDS) {
+            const uint32_t* xp = static_cast<const uint32_t*>(P.x);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+                xw[i] = wm0 + 32 * i + lc < rows_here ? xp[xwo[i] + kc] : 0u;
+            if (noisy) xbits = xvalid ? xp[2 * xoff + kc] >> xk : 0u;
+        } else if (xvalid && xal && k + KPT <= b) {
+            if constexpr (XFMT == HSES_FMT_F32) {
+                const float4* xp = reinterpret_cast<const float4*>(static_cast<const float*>(P.x) + xoff + k);
+#pragma unroll
+                for (int q = 0; q < KPT / 4; ++q) *reinterpret_cast<float4*>(xv + 4 * q) = xp[q];
+            } else {
+                const uint4* xp = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(P.x) + xoff + k);
+#pragma unroll
+                for (int q = 0; q < KPT / 8; ++q) {
+                    const uint4 u = xp[q];
+                    const uint32_t w4[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        xv[8 * q + 2 * e] = __uint_as_float(w4[e] << 16);
+                        xv[8 * q + 2 * e + 1] = __uint_as_float(w4[e] & 0xffff0000u);
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < KPT; ++i)
+                xv[i] = (xvalid && k + i < b) ? x_at<XFMT>(P.x, xoff, k + i) : 0.0f;
+        }
+        // W parts of the chunk: [part][o0 ..][32], whole 64-byte rows
+#pragma unroll
+        for (int j = 0; j < WPC; ++j) {
+            const int32_t e = tid + KF_THREADS * j, p = e / (BN * 4), q = e % (BN * 4);
+            if (BN * 12 % KF_THREADS == 0 || e < BN * 12)
+                wv[j] = reinterpret_cast<const u32x4*>(Wp)[((int64_t)(kc * 3 + p) * a_pad + o0) * 4 + q];
+        }
+        if (noisy) {
+#pragma unroll
+            for (int j = 0; j < BPT; ++j)
+                if (KF_THREADS * j < bch)  // uniform
+                    bv[j] = Fm[b_ok(j, kc) ? boff[j] + kc * KF_BK * r : 0];
+        }
+    };
+    auto store_chunk = [&](int32_t kc) {
+#pragma unroll
+        for (int q = 0; q < (XLDS ? KPT / 8 : 0); ++q) {
+            uint32_t d[3][4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                uint32_t p[3];
+                const float lo = xv[8 * q + 2 * u], hi = xv[8 * q + 2 * u + 1];
+                if constexpr (NP == 3) split3(lo, hi, p);
+                else p[0] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
+#pragma unroll
+                for (int w = 0; w < NP; ++w) d[w][u] = p[w];
+            }
+            const int s = slot_of(xr, (xk >> 3) + q);
+#pragma unroll
+            for (int w = 0; w < NP; ++w)
+                *reinterpret_cast<uint4*>(Xs + (w * BM + xr) * KF_BK + 8 * s) =
+                    uint4{d[w][0], d[w][1], d[w][2], d[w][3]};
+        }
+#pragma unroll
+        for (int j = 0; j < WPC; ++j) {
+            const int32_t e = tid + KF_THREADS * j;
+            if (BN * 12 % KF_THREADS == 0 || e < BN * 12) reinterpret_cast<u32x4*>(Ws)[e] = wv[j];
+        }
+        if (noisy) {
+#pragma unroll
+            for (int j = 0; j < BPT; ++j) {
+                const int32_t e = tid + KF_THREADS * j;
+                if (KF_THREADS * j < bch && e < bch) Bc[e] = b_ok(j, kc) ? bv[j] : 0.0f;
+            }
+        }
+    };
+
+    // acc: the products of the leading parts; low: those of the others, 2^-8 of
+    // them and less, so that the rounding of their many sums does not count
+    f32x16 acc[MI][NJ], low[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.0f;
+    float xb[RK];  // this thread's share of (x B_m) for row xr
+#pragma unroll
+    for (int c = 0; c < RK; ++c) xb[c] = 0.0f;
+
+    const int32_t nch = (b + KF_BK - 1) / KF_BK;
+    load_chunk(0);
+    for (int32_t kc = 0; kc < nch; ++kc) {
+        if (kc) __syncthreads();  // every wave is past its reads of chunk kc - 1
+        store_chunk(kc);
+        __syncthreads();
+        if (noisy) {
+            // x B_m over this thread's KPT k, fp32 in ascending k
+            const float* bs = Bc + (xlm * KF_BK + xk) * RK;
+#pragma unroll
+            for (int i = 0; i < KPT; ++i) {
+                float be[RK];
+                if constexpr (RK == 1) {
+                    be[0] = bs[i];
+                } else {
+#pragma unroll
+                    for (int q = 0; q < RK / 4; ++q)
+                        *reinterpret_cast<float4*>(be + 4 * q) =
+                            *reinterpret_cast<const float4*>(bs + i * RK + 4 * q);
+                }
+                const float v = XLDS ? xv[i] : (float)((xbits >> i) & 1u);
+#pragma unroll
+                for (int c = 0; c < RK; ++c) xb[c] = __builtin_fmaf(v, be[c], xb[c]);
+            }
+        }
+        uint32_t xc[MI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) xc[i] = XLDS ? 0u : xw[i];
+        if (kc + 1 < nch) load_chunk(kc + 1);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            u16x8 af[MI][NP], bf[NJ][3];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int row = wn0 + 32 * j + lc, s = slot_of(row, 2 * ks + kh);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) bf[j][p] = lds_u16x8(Ws + (p * BN + row) * KF_BK + 8 * s);
+            }
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                if constexpr (XLDS) {
+                    const int row = wm0 + 32 * i + lc, s = slot_of(row, 2 * ks + kh);
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) af[i][p] = lds_u16x8(Xs + (p * BM + row) * KF_BK + 8 * s);
+                } else {
+                    af[i][0] = expand_bits((xc[i] >> (16 * ks + 8 * kh)) & 0xffu);
+                }
+            }
+            // the products down to 2^-16 of the largest: x_p w_q, p + q <= 2
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int q = 0; q < 3 - p; ++q)
+#pragma unroll
+                    for (int i = 0; i < MI; ++i)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) {
+                            if (p + q == 0) acc[i][j] = mfma_bf(af[i][p], bf[j][q], acc[i][j]);
+                            else low[i][j] = mfma_bf(af[i][p], bf[j][q], low[i][j]);
+                        }
+        }
+    }
+
+    // ---- epilogue: y = x W^T + (x B_m) A_m^T -----------------------------------------
+    __syncthreads();
+    float* XBs = reinterpret_cast<float*>(smem);  // [BM][RK]; the staging buffers are free
+    if (noisy) {
+#pragma unroll
+        for (int c = 0; c < RK; ++c) {
+            float v = xb[c] + __shfl_xor(xb[c], 1);  // the row's k shares
+            if constexpr (TPR == 4) v += __shfl_xor(v, 2);
+            if (xk == 0) XBs[xr * RK + c] = v;
+        }
+        __syncthreads();
+    }
+    auto add_noise = [&](float yv, int32_t row, int32_t col) {
+        const float* ar = As + ((size_t)rlm[row] * BN + col) * RK;
+        float z = 0.0f;
+#pragma unroll
+        for (int c = 0; c < RK; ++c) z = __fadd_rn(z, __fmul_rn(XBs[row * RK + c], ar[c]));
+        return __fadd_rn(yv, z);
+    };
+    // accumulator element e of lane l: row 8 (e / 4) + 4 kh + e % 4 of the
+    // 32-row tile, column lc
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int32_t row = wm0 + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
+            if (row >= rows_here) continue;
+            float* yrow = P.y + yoffs[row];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int32_t col = wn0 + 32 * j + lc;
+                if (col >= ct) continue;
+                const float yv = __fadd_rn(acc[i][j][e], low[i][j][e]);
+                bad |= !(fabsf(yv) < INFINITY);
+                yrow[col] = noisy ? add_noise(yv, row, col) : yv;
+            }
+        }
+    // A part of an infinity, a NaN or a magnitude that rounds up to infinity is
+    // not finite and leaves its row or column of sums so: the wave then forms
+    // its outputs again with plain fp32 chains, which give what fp32 gives.
+    if (__any(bad)) {
+#pragma unroll 1
+        for (int32_t e = lane; e < WM * WN; e += 64) {
+            const int32_t row = wm0 + e / WN, col = wn0 + e % WN;
+            if (row >= rows_here || col >= ct) continue;
+            const float* w = P.W + (P.tmm ? o0 + col : (int64_t)(o0 + col) * b);
+            const int64_t wk = P.tmm ? P.a : 1, xo = xoffs[row];
+            float yv = 0.0f;
+#pragma unroll 1
+            for (int32_t k = 0; k < b; ++k) yv = __builtin_fmaf(x_at<XFMT>(P.x, xo, k), w[k * wk], yv);
+            P.y[yoffs[row] + col] = noisy ? add_noise(yv, row, col) : yv;
+        }
+    }
 }
 
 // ---- k_gemm_f32 ------------------------------------------------------------------
@@ -339,14 +720,28 @@ __global__ __launch_bounds__(KF_THREADS) void k_gemm_f32(LinParams P, const floa
 
 static int32_t f32_bn(int32_t a) { return a <= 32 ? 32 : a <= 64 ? 64 : 128; }
 static int32_t f32_rk(int32_t r) { return r <= 1 ? 1 : r <= 4 ? 4 : r <= 8 ? 8 : 16; }
+static int32_t f32_pad(int32_t a) { return (a + f32_bn(a) - 1) / f32_bn(a) * f32_bn(a); }
 
-// Most members a 128-row tile (starting at a multiple of 128) can touch.
-static int32_t f32_nm_max(int32_t R, int32_t n) {
+// k_gemm_f32s takes do_Tmm (which k_gemm_f32 does not) and do_mm with at least
+// 256 outputs, over more than two K chunks (at b <= 64 a call is bound by its x
+// and y bytes).  Narrower do_mm outputs are the spiking layers': their currents
+// stay on the fp32 chain, because a current at the LIF threshold would spike or
+// not with the order of its sum.  The rule is the same for every x format
+// (binary inputs give the same bits in all of them).
+static bool f32_split_shape(int32_t a, int32_t b, bool tmm) {
+    return b > 2 * KF_BK && (tmm || a >= 256);
+}
+static size_t f32_w_bytes(int32_t a, int32_t b) {
+    return b > 2 * KF_BK ? (size_t)((b + KF_BK - 1) / KF_BK) * 3 * f32_pad(a) * KF_BK * 2 : 0;
+}
+
+// Most members a bm-row tile (starting at a multiple of bm) can touch.
+static int32_t f32_nm_max(int32_t bm, int32_t R, int32_t n) {
     int32_t nm;
-    if (R % KF_BM == 0) nm = 1;
-    else if (R > KF_BM) nm = 2;
-    else if (KF_BM % R == 0) nm = KF_BM / R;
-    else nm = (KF_BM - 1) / R + 2;
+    if (R % bm == 0) nm = 1;
+    else if (R > bm) nm = 2;
+    else if (bm % R == 0) nm = bm / R;
+    else nm = (bm - 1) / R + 2;
     return std::min(nm, n);
 }
 
@@ -363,25 +758,38 @@ static bool factor_rows(const LinParams& P, int32_t* rc_out, int32_t* groups) {
     return true;
 }
 
-// The tiling of one call (shape only).
+// The tiling of one call (shape only).  split: k_gemm_f32s.
 struct F32Plan {
-    int32_t bn, rk, nm, bch;
-    size_t lds, f_bytes;
+    bool split;
+    int32_t bm, bn, rk, bch;
+    size_t lds, f_bytes, w_bytes;
 };
 
-static bool f32_plan(const LinParams& P, F32Plan* pl) {
-    if (P.math != HSES_MATH_F32 || P.tmm || P.r > KF_RMAX || P.r < 0) return false;
+static bool f32_plan(const LinParams& P, bool split, F32Plan* pl) {
+    if (P.math != HSES_MATH_F32 || P.r > KF_RMAX || P.r < 0) return false;
+    if (split ? !f32_split_shape(P.a, P.b, P.tmm) : P.tmm) return false;
     const int32_t r = P.r;
+    pl->split = split;
     pl->bn = f32_bn(P.a);
+    pl->bm = KF_BM;
+    // split: 64 x 64 tiles while 128-row tiles would leave CUs without one (256 CUs)
+    if (split && pl->bn >= 64 && (P.total + 127) / 128 * (f32_pad(P.a) / pl->bn) < 256)
+        pl->bm = pl->bn = 64;
     pl->rk = f32_rk(r);
-    pl->nm = f32_nm_max(P.R, P.n);
-    const size_t bch = r > 0 ? (size_t)pl->nm * KF_BK * pl->rk : 0;
-    if (bch > 8 * KF_THREADS) return false;  // BPT values per thread
+    const int32_t nm = f32_nm_max(pl->bm, P.R, P.n);
+    const size_t bch = r > 0 ? (size_t)nm * KF_BK * pl->rk : 0;
+    if (bch > (size_t)(split ? KS_BPT : 8) * KF_THREADS) return false;  // BPT values per thread
     pl->bch = (int32_t)bch;
-    const size_t a_lds = r > 0 ? (size_t)pl->nm * pl->bn * pl->rk : 0;
+    const size_t a_lds = r > 0 ? (size_t)nm * pl->bn * pl->rk : 0;
     if (a_lds > KF_AMAX) return false;
-    const size_t nbuf = P.b > KF_BK ? 2 : 1;  // staging buffers (k_gemm_f32)
-    pl->lds = (nbuf * ((size_t)(KF_BM + pl->bn) * KF_XP + bch) + a_lds) * 4;
+    if (split) {
+        const size_t parts = P.x_fmt == HSES_FMT_F32 ? 3 : P.x_fmt == HSES_FMT_BF16 ? 1 : 0;
+        pl->lds = (parts * pl->bm + 3 * pl->bn) * KF_BK * 2 + bch * 4 + (size_t)pl->bm * 20 + a_lds * 4;
+    } else {
+        const size_t nbuf = P.b > KF_BK ? 2 : 1;  // staging buffers (k_gemm_f32)
+        pl->lds = (nbuf * ((size_t)(KF_BM + pl->bn) * KF_XP + bch) + a_lds) * 4;
+    }
+    pl->w_bytes = split ? f32_w_bytes(P.a, P.b) : 0;
     pl->f_bytes = 0;
     if (r > 0) {
         int32_t rc, groups;
@@ -391,16 +799,26 @@ static bool f32_plan(const LinParams& P, F32Plan* pl) {
     return true;
 }
 
-int launch_factors(LinParams& P, DeviceState* st, hipStream_t s, float* F) {
-    int32_t rc, groups;
-    if (P.r < 1 || !factor_rows(P, &rc, &groups)) return HSES_ERR_UNSUPPORTED;
-    int e = get_jump_table(st, (int64_t)rc * P.r, groups, &P.jump);
-    if (e) return e;
-    const int64_t blocks = ((int64_t)P.n * groups + 255) / 256;
+// k_factors: the factor rows (rank 0: none) into F, the split of W into Wp (or NULL).
+static int launch_factors_w(LinParams& P, DeviceState* st, hipStream_t s, float* F, uint16_t* Wp) {
+    int32_t rc = 1, groups = 0;
+    if (P.r > 0) {
+        if (!factor_rows(P, &rc, &groups)) return HSES_ERR_UNSUPPORTED;
+        int e = get_jump_table(st, (int64_t)rc * P.r, groups, &P.jump);
+        if (e) return e;
+    }
+    const int64_t fblocks = ((int64_t)P.n * groups + 255) / 256;
+    const int64_t pieces = Wp ? (int64_t)((P.b + KF_BK - 1) / KF_BK) * f32_pad(P.a) * 4 : 0;
+    const int64_t blocks = fblocks + (pieces + 255) / 256;
     if (blocks > INT32_MAX) return set_error(HSES_ERR_INVALID_ARG, "too many factor rows");
-    hipLaunchKernelGGL(k_factors, dim3((uint32_t)blocks), dim3(256), 0, s, P, rc, groups, F);
+    hipLaunchKernelGGL(k_factors, dim3((uint32_t)blocks), dim3(256), 0, s, P, rc, groups, F,
+                       (int32_t)fblocks, Wp, f32_pad(P.a));
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
+}
+
+int launch_factors(LinParams& P, DeviceState* st, hipStream_t s, float* F) {
+    return P.r < 1 ? HSES_ERR_UNSUPPORTED : launch_factors_w(P, st, s, F, nullptr);
 }
 
 size_t linear_f32_workspace(int32_t a, int32_t b, int32_t r, int32_t n, int32_t rows_per_member,
@@ -408,26 +826,27 @@ size_t linear_f32_workspace(int32_t a, int32_t b, int32_t r, int32_t n, int32_t 
     (void)rows_per_member;
     (void)n_time;
     if (math != HSES_MATH_F32 || a < 1 || b < 1 || n < 1 || r < 0 || r > KF_RMAX) return 0;
-    return align16((size_t)n * (a + b) * r * 4);
+    return align16((size_t)n * (a + b) * r * 4) + f32_w_bytes(a, b);
+}
+
+template <typename Kern, typename... Args>
+static int launch_f32(Kern kern, size_t lds, dim3 grid, hipStream_t s, Args... args) {
+    if (lds > 64 * 1024)
+        HSES_CHECK_HIP(hipFuncSetAttribute((const void*)kern,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, grid, dim3(KF_THREADS), lds, s, args...);
+    HSES_CHECK_HIP(hipGetLastError());
+    return HSES_OK;
 }
 
 template <int XFMT, int NT>
 static int launch_gemm_rk(const LinParams& P, const F32Plan& pl, hipStream_t s, const float* F,
                           dim3 grid) {
-    auto launch = [&](auto kern) -> int {
-        if (pl.lds > 64 * 1024)
-            HSES_CHECK_HIP(hipFuncSetAttribute((const void*)kern,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)pl.lds));
-        hipLaunchKernelGGL(kern, grid, dim3(KF_THREADS), pl.lds, s, P, F, pl.bch);
-        HSES_CHECK_HIP(hipGetLastError());
-        return HSES_OK;
-    };
     switch (pl.rk) {
-        case 1: return launch(k_gemm_f32<XFMT, NT, 1>);
-        case 4: return launch(k_gemm_f32<XFMT, NT, 4>);
-        case 8: return launch(k_gemm_f32<XFMT, NT, 8>);
-        default: return launch(k_gemm_f32<XFMT, NT, 16>);
+        case 1: return launch_f32(k_gemm_f32<XFMT, NT, 1>, pl.lds, grid, s, P, F, pl.bch);
+        case 4: return launch_f32(k_gemm_f32<XFMT, NT, 4>, pl.lds, grid, s, P, F, pl.bch);
+        case 8: return launch_f32(k_gemm_f32<XFMT, NT, 8>, pl.lds, grid, s, P, F, pl.bch);
+        default: return launch_f32(k_gemm_f32<XFMT, NT, 16>, pl.lds, grid, s, P, F, pl.bch);
     }
 }
 
@@ -441,20 +860,51 @@ static int launch_gemm_bn(const LinParams& P, const F32Plan& pl, hipStream_t s, 
     }
 }
 
+template <int XFMT, int BM, int BN>
+static int launch_split_rk(const LinParams& P, const F32Plan& pl, hipStream_t s, const float* F,
+                           const uint16_t* Wp, dim3 grid) {
+    const int32_t ap = f32_pad(P.a);
+    switch (pl.rk) {
+        case 1: return launch_f32(k_gemm_f32s<XFMT, BM, BN, 1>, pl.lds, grid, s, P, F, Wp, ap, pl.bch);
+        case 4: return launch_f32(k_gemm_f32s<XFMT, BM, BN, 4>, pl.lds, grid, s, P, F, Wp, ap, pl.bch);
+        case 8: return launch_f32(k_gemm_f32s<XFMT, BM, BN, 8>, pl.lds, grid, s, P, F, Wp, ap, pl.bch);
+        default: return launch_f32(k_gemm_f32s<XFMT, BM, BN, 16>, pl.lds, grid, s, P, F, Wp, ap, pl.bch);
+    }
+}
+
+template <int XFMT>
+static int launch_split_bn(const LinParams& P, const F32Plan& pl, hipStream_t s, const float* F,
+                           const uint16_t* Wp, dim3 grid) {
+    if (pl.bm == 64) return launch_split_rk<XFMT, 64, 64>(P, pl, s, F, Wp, grid);
+    switch (pl.bn) {
+        case 32: return launch_split_rk<XFMT, 128, 32>(P, pl, s, F, Wp, grid);
+        case 64: return launch_split_rk<XFMT, 128, 64>(P, pl, s, F, Wp, grid);
+        default: return launch_split_rk<XFMT, 128, 128>(P, pl, s, F, Wp, grid);
+    }
+}
+
 int launch_linear_f32(LinParams& P, DeviceState* st, hipStream_t s, void* work, size_t work_bytes) {
     F32Plan pl;
-    if (!f32_plan(P, &pl)) return HSES_ERR_UNSUPPORTED;
-    if (pl.lds > st->max_lds) return HSES_ERR_UNSUPPORTED;
-    if (P.r > 0 && (!work || work_bytes < pl.f_bytes)) return HSES_ERR_UNSUPPORTED;
-    const int64_t row_tiles = (P.total + KF_BM - 1) / KF_BM;
-    const int64_t tiles = row_tiles * ((P.a + pl.bn - 1) / pl.bn);
+    auto fits = [&](bool split) {
+        return f32_plan(P, split, &pl) && pl.lds <= st->max_lds &&
+               (pl.f_bytes + pl.w_bytes == 0 || (work && work_bytes >= pl.f_bytes + pl.w_bytes)) &&
+               (!split || reinterpret_cast<uintptr_t>(work) % 16 == 0);
+    };
+    if (!fits(true) && !fits(false)) return HSES_ERR_UNSUPPORTED;
+    const int64_t tiles = (P.total + pl.bm - 1) / pl.bm * ((P.a + pl.bn - 1) / pl.bn);
     if (tiles > INT32_MAX) return set_error(HSES_ERR_INVALID_ARG, "too many output rows");
     float* F = static_cast<float*>(work);
-    if (P.r > 0) {
-        const int rc = launch_factors(P, st, s, F);
+    uint16_t* Wp = pl.split ? reinterpret_cast<uint16_t*>(static_cast<char*>(work) + pl.f_bytes) : nullptr;
+    if (P.r > 0 || Wp) {
+        const int rc = launch_factors_w(P, st, s, F, Wp);
         if (rc) return rc;
     }
     const dim3 grid((uint32_t)tiles);
+    if (pl.split) switch (P.x_fmt) {
+        case HSES_FMT_BITS: return launch_split_bn<HSES_FMT_BITS>(P, pl, s, F, Wp, grid);
+        case HSES_FMT_BF16: return launch_split_bn<HSES_FMT_BF16>(P, pl, s, F, Wp, grid);
+        default: return launch_split_bn<HSES_FMT_F32>(P, pl, s, F, Wp, grid);
+    }
     switch (P.x_fmt) {
         case HSES_FMT_BITS: return launch_gemm_bn<HSES_FMT_BITS>(P, pl, s, F, grid);
         case HSES_FMT_BF16: return launch_gemm_bn<HSES_FMT_BF16>(P, pl, s, F, grid);

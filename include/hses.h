@@ -212,7 +212,8 @@ int hses_lif_scan(const float *d_cur, const float *d_v0, int32_t T, int64_t rows
  * M*stride) and the time-inner layout (each row's T entries adjacent:
  * plane >= a row, stride >= T*plane) are both accepted, for x, y and spikes.
  * sigma=0 or rank=0 gives the clean x W^T.
- * d_work must hold hses_perturbed_linear_workspace(...) bytes (a bf16 copy of W
+ * d_work must hold hses_perturbed_linear_workspace(...) bytes (a bf16 copy of W, or
+ * for fp32 math its bf16 parts, the members' factor rows at small ranks
  * and, for large ranks, one per-workgroup staging slot for a pair's B factor;
  * the (n, b, r) factor tensor itself is never materialised).  Large ranks
  * (r a multiple of 16, r <= 128, a <= 128) need math = HSES_MATH_BF16.  With

@@ -1,0 +1,90 @@
+"""The fp32 forward on split operands (k_gemm_f32s: do_Tmm, and do_mm with at
+least 256 outputs, over inputs more than 64 wide) against float64.
+
+Bound: a product of two bf16 parts is exact in the fp32 accumulator, the
+products left out are below 2^-25 of |x w|, and a running sum is rounded at most
+once per k and part product plus the few roundings that put the sums together;
+each is at most half an ulp of a partial sum below sum |x w|.  Rounding errors
+of K terms grow like sqrt(K): 2^-24 (4 sqrt(K) + 8) of the sum of |terms|."""
+import numpy as np
+import pytest
+import torch
+
+from hyperscalees_amd._lib import FMT_BF16, FMT_BITS, FMT_F32
+from tests import oracle_lib as O
+from tests.test_gpu_linear import KEY, factors, pack_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(x3, W, A, B, rpm, tmm):
+    """float64 y and sum of |terms|; W is (out, in), or (in, out) for do_Tmm."""
+    Wd = (W.T if tmm else W).astype(np.float64)
+    y, s = x3 @ Wd.T, np.abs(x3) @ np.abs(Wd).T
+    for m in range(A.shape[0] if A is not None else 0):
+        i, o = (A[m], B[m]) if tmm else (B[m], A[m])
+        rows = slice(m * rpm, (m + 1) * rpm)
+        y[:, rows] += (x3[:, rows] @ i.astype(np.float64)) @ o.astype(np.float64).T
+        s[:, rows] += (np.abs(x3[:, rows]) @ np.abs(i)) @ np.abs(o).T
+    return y, s
+
+
+@pytest.mark.parametrize("n,rpm,T,out,inp,r,tid_lo,tmm,fmt", [
+    (2, 300, 1, 256, 65, 1, 0, 0, FMT_F32),      # shortest split K, a ragged last chunk
+    (5, 131, 1, 257, 96, 2, 1, 0, FMT_F32),      # one column past a tile, odd first member
+    (3, 37, 3, 1000, 99, 4, 0, 0, FMT_F32),      # unaligned rows, members straddle tiles
+    (2, 512, 40, 300, 784, 4, 1, 0, FMT_BITS),   # 128-row tiles, bit-packed
+    (40, 257, 1, 384, 160, 8, 0, 0, FMT_BF16),   # 128-row tiles, bf16 x
+    (300, 128, 1, 256, 72, 16, 0, 0, FMT_F32),   # largest rank
+    (1, 1, 1, 256, 66, 0, 0, 0, FMT_F32),        # one row, no noise
+    (4, 50, 1, 10, 100, 4, 3, 1, FMT_F32),       # do_Tmm, 32-column tile
+    (70, 500, 1, 33, 130, 1, 0, 1, FMT_F32),     # do_Tmm, 64-column tile, 128 rows
+    (9, 40, 2, 70, 256, 1, 1, 1, FMT_BF16),      # do_Tmm, two column tiles
+    (6, 64, 2, 130, 200, 2, 0, 1, FMT_BITS),
+])
+def test_split_against_float64(hses_gpu, n, rpm, T, out, inp, r, tid_lo, tmm, fmt):
+    rng = np.random.default_rng(out + inp + r)
+    x3 = rng.standard_normal((T, n * rpm, inp)).astype(np.float32)
+    x3 *= np.exp2(rng.integers(-12, 13, inp)).astype(np.float32)   # no common scale
+    if fmt == FMT_BITS:
+        x3 = (x3 > 0).astype(np.float32)
+        xt = pack_bits(x3)
+    elif fmt == FMT_BF16:
+        xt = torch.from_numpy(x3).to(torch.bfloat16).cuda()
+        x3 = xt.float().cpu().numpy()
+    else:
+        xt = torch.from_numpy(x3).cuda()
+    shape = (inp, out) if tmm else (out, inp)
+    W = (rng.standard_normal(shape) / np.sqrt(inp)).astype(np.float32)
+    A = B = None
+    if r:
+        A, B = factors(0.2, r, n, tid_lo, *shape)
+    ref, s = reference(x3.astype(np.float64), W, A, B, rpm, tmm)
+    f = hses_gpu.perturbed_linear_t if tmm else hses_gpu.perturbed_linear
+    y = f(xt, torch.from_numpy(W).cuda(), KEY, r, 0.2 if r else 0.0, 0, 0, tid_lo, n, rpm, x_fmt=fmt,
+          n_time=T).cpu().numpy().reshape(ref.shape)
+    # x B_m and (x B_m) A_m^T run as fp32 chains of inp and r terms
+    tol = 2.0 ** -24 * (4 * np.sqrt(inp + r) + 8)
+    err = (np.abs(y - ref) / s).max()
+    assert err <= tol, f"error {err:.2e} of the sum of |terms|, bound {tol:.2e}"
+
+
+def test_split_values_without_parts(hses_gpu):
+    """Infinities, NaN and magnitudes that round up past bf16's range give what an
+    fp32 chain gives, and leave the other rows and columns alone."""
+    rng = np.random.default_rng(3)
+    n, inp, out = 300, 100, 300
+    x = rng.standard_normal((n, inp)).astype(np.float32)
+    W = rng.standard_normal((out, inp)).astype(np.float32)
+    x[3, 7], x[140, 0], x[141, 99], x[200, 5] = np.inf, np.nan, -np.inf, np.float32(3.4e38)
+    x[200, :5], x[200, 6:] = 0.0, 0.0
+    W[17, 50], W[280, 3], W[:, 5] = np.inf, np.nan, np.clip(W[:, 5], -0.9, 0.9)
+    y = hses_gpu.perturbed_linear(torch.from_numpy(x).cuda(), torch.from_numpy(W).cuda(), KEY, 0, 0.0, 0,
+                                  0, 0, n, 1).cpu().numpy().reshape(n, out)
+    with np.errstate(all="ignore"):
+        ref = x.astype(np.float64) @ W.astype(np.float64).T
+        s = np.abs(x).astype(np.float64) @ np.abs(W).astype(np.float64).T
+    fin = np.isfinite(ref)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
+    np.testing.assert_array_equal(y[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
+    assert (np.abs(y[fin] - ref[fin]) <= 2.0 ** -24 * (4 * np.sqrt(inp) + 8) * s[fin]).all()
