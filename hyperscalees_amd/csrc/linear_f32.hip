@@ -108,14 +108,19 @@ __device__ __forceinline__ void split_w(const LinParams& P, uint16_t* Wp, int32_
 // ---- k_factors -------------------------------------------------------------------
 // F[m] = the member's (a + b) x r stream rows as drawn, except that the
 // rows carrying sign * sigma / sqrt(r) are scaled: do_mm's A rows [b, a + b),
-// do_Tmm's input-side rows [a, a + b) (with a the output width).  A thread
-// draws rows [q rc, q rc + rc) of one member after one jump to the group's start.
-// Blocks from fblocks on split W for k_gemm_f32 (Wp, NULL without one): with
+// do_Tmm's input-side rows [a, a + b) (with a the output width).  Members 2p
+// and 2p + 1 share pair p's normals with the scaled rows negated, so a thread
+// draws rows [q rc, q rc + rc) of one pair after one jump to the group's start
+// and stores them for both members.  Bound by the draw's vector instructions
+// (about 106 per normal): drawing per pair and not per member halves them
+// (4096 members, 2048 rows, rank 1: 42.8 -> FACT_US us).
+// Blocks from fblocks on split W for k_gemm_f32s (Wp, NULL without one): with
 // a_pad output rows, [k chunk of 32][part][output row][32], the 16-byte pieces
-// of a row swizzled as k_gemm_f32 reads them from LDS (slot_of), zero past a
+// of a row swizzled as k_gemm_f32s reads them from LDS (slot_of), zero past a
 // and b.  A block takes 256 pieces of 8 k.
-__global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_t groups,
-                                                 float* __restrict__ F, int32_t fblocks,
+// vec: every group starts 16-byte aligned.
+__global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_t groups, int32_t pairs,
+                                                 float* __restrict__ F, int32_t vec, int32_t fblocks,
                                                  uint16_t* __restrict__ Wp, int32_t a_pad) {
     __shared__ BmTables t;
     if ((int32_t)blockIdx.x >= fblocks) {
@@ -125,18 +130,44 @@ __global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_
     load_bm_tables(&t, P.tables);
     __syncthreads();
     const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (item >= (int64_t)P.n * groups) return;
-    const int32_t m = (int32_t)(item / groups), q = (int32_t)(item % groups);
+    if (item >= (int64_t)pairs * groups) return;
+    const int32_t p = (int32_t)(item / groups), q = (int32_t)(item % groups);
     const int32_t r = P.r, rows = P.a + P.b, row0 = q * rc;
+    const int32_t tid = 2 * (P.tid_lo / 2 + p), m = tid - P.tid_lo;  // the pair's even member (-1: not ours)
     float sign;
-    const uint64_t seed = member_seed(P.key, P.epoch, P.nreuse, P.tid_lo + m, &sign);
-    const float sc = sign * P.bs;
+    const uint64_t seed = member_seed(P.key, P.epoch, P.nreuse, tid, &sign);
     uint64_t s = row_start_state(seed, q, P.jump);
     const NoiseCtx ctx{&t, P.log_exc, P.cos_exc};
-    float* dst = F + ((int64_t)m * rows + row0) * r;
+    float* even = F + ((int64_t)m * rows + row0) * r;
+    float* odd = even + (int64_t)rows * r;
+    const bool we = m >= 0, wo = m + 1 < P.n;
     const int32_t split = ((P.tmm ? P.a : P.b) - row0) * r;  // normals before the first scaled row
-    bm_run(s, min(rc, rows - row0) * r, ctx,
-           [&](int32_t i, float v) { dst[i] = i >= split ? v * sc : v; });
+    auto one = [&](int32_t i, float v) {
+        const float e = i >= split ? v * P.bs : v;
+        if (we) even[i] = e;
+        if (wo) odd[i] = i >= split ? -e : e;
+    };
+    bm_run2<4>(
+        s, min(rc, rows - row0) * r, ctx,
+        [&](int32_t i, const float* v) {
+            if (!vec) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) one(i + u, v[u]);
+                return;
+            }
+            float4 e, o;
+            float* ep = reinterpret_cast<float*>(&e);
+            float* op = reinterpret_cast<float*>(&o);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool sc = i + u >= split;
+                ep[u] = sc ? v[u] * P.bs : v[u];
+                op[u] = sc ? -ep[u] : ep[u];
+            }
+            if (we) *reinterpret_cast<float4*>(even + i) = e;
+            if (wo) *reinterpret_cast<float4*>(odd + i) = o;
+        },
+        one);
 }
 
 // ---- k_gemm_f32s -----------------------------------------------------------------
@@ -745,12 +776,19 @@ static int32_t f32_nm_max(int32_t bm, int32_t R, int32_t n) {
     return std::min(nm, n);
 }
 
-// Rows per generating thread: up to 32 normals, fewer while that leaves under
-// 64k threads; at least enough for the jump tables' row count.
+static int32_t factor_pairs(const LinParams& P) {
+    return (int32_t)(((int64_t)P.tid_lo + P.n - 1) / 2 - P.tid_lo / 2 + 1);
+}
+
+// Rows per generating thread: up to 16 normals, fewer while that leaves under
+// 128k threads (two waves per SIMD); at least enough for the jump tables' row
+// count.  1024 pairs x 1024 rows at rank 1: 24.1 us with 64k threads (16 normals
+// each), 21.5 with 128k, 33 with 256k (4 normals: the jumps dominate); 2048 x
+// 2048: 47 us at 32 normals per thread, 37 at 16, 44 at 8.
 static bool factor_rows(const LinParams& P, int32_t* rc_out, int32_t* groups) {
     const int32_t r = P.r, rows = P.a + P.b;
-    int32_t rc = std::max(1, 32 / r);
-    while (rc > 1 && (int64_t)P.n * ((rows + rc - 1) / rc) < 65536) rc = std::max(1, rc / 2);
+    int32_t rc = std::max(1, 16 / r);
+    while (rc > 1 && (int64_t)factor_pairs(P) * ((rows + rc - 1) / rc) < 131072) rc = std::max(1, rc / 2);
     rc = std::max<int32_t>(rc, (int32_t)((rows + kJumpMaxRows - 1) / kJumpMaxRows));
     if ((int64_t)rc * r > kJumpMaxL) return false;
     *rc_out = rc;
@@ -807,12 +845,15 @@ static int launch_factors_w(LinParams& P, DeviceState* st, hipStream_t s, float*
         int e = get_jump_table(st, (int64_t)rc * P.r, groups, &P.jump);
         if (e) return e;
     }
-    const int64_t fblocks = ((int64_t)P.n * groups + 255) / 256;
+    const int32_t pairs = factor_pairs(P);
+    const int32_t vec = reinterpret_cast<uintptr_t>(F) % 16 == 0 && (int64_t)(P.a + P.b) * P.r % 4 == 0 &&
+                        rc * P.r % 4 == 0;
+    const int64_t fblocks = ((int64_t)pairs * groups + 255) / 256;
     const int64_t pieces = Wp ? (int64_t)((P.b + KF_BK - 1) / KF_BK) * f32_pad(P.a) * 4 : 0;
     const int64_t blocks = fblocks + (pieces + 255) / 256;
     if (blocks > INT32_MAX) return set_error(HSES_ERR_INVALID_ARG, "too many factor rows");
-    hipLaunchKernelGGL(k_factors, dim3((uint32_t)blocks), dim3(256), 0, s, P, rc, groups, F,
-                       (int32_t)fblocks, Wp, f32_pad(P.a));
+    hipLaunchKernelGGL(k_factors, dim3((uint32_t)blocks), dim3(256), 0, s, P, rc, groups,
+                       pairs, F, vec, (int32_t)fblocks, Wp, f32_pad(P.a));
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }
