@@ -163,7 +163,9 @@ int launch_linear_small(LinParams& P, DeviceState* st, hipStream_t s);
 int launch_linear_f32(LinParams& P, DeviceState* st, hipStream_t s, void* work, size_t work_bytes);
 // Every member's (a + b) x r factor rows into F (n (a + b) r floats), the
 // scaled role's rows (do_mm: A; do_Tmm: the input side) times sign * sigma / sqrt(r).
-int launch_factors(LinParams& P, DeviceState* st, hipStream_t s, float* F);
+// With Fb (rank 1; 8-byte aligned, a + b, b and the input side's first row
+// multiples of 4) the input side's rows go to Fb as bf16, n b values.
+int launch_factors(LinParams& P, DeviceState* st, hipStream_t s, float* F, uint16_t* Fb = nullptr);
 // bf16 math, outputs >= 256 wide, rank <= 4: the bf16 MFMA GEMM with x B_m
 // fused (linear_bf16.hip); its workspace, 0 when it does not apply.
 int launch_linear_bf16(LinParams& P, DeviceState* st, hipStream_t s, void* work, size_t work_bytes,

@@ -72,10 +72,10 @@ __device__ __forceinline__ void split3(float lo, float hi, uint32_t (&p)[3]) {
     p[2] = pack_bf16x2(l1 - __uint_as_float(p[1] << 16), h1 - __uint_as_float(p[1] & 0xffff0000u));
 }
 
-// Slot of 16-byte piece s (8 k) of row `row` in its 64-byte LDS row: a lane of
-// a quarter-wave reads the same piece of eight consecutive rows, which the XOR
-// puts on distinct banks.
-__device__ __forceinline__ int slot_of(int row, int s) { return s ^ ((row >> 1) & 3); }
+// Slot of 16-byte piece s (8 k) of row `row` in its 64-byte LDS row.  The lanes of
+// a 16-byte read are served 16 at a time over 64 banks; they read one piece of
+// 16 rows, four of each row / 4 class mod 4, which the XOR spreads over the banks.
+__device__ __forceinline__ int slot_of(int row, int s) { return s ^ ((row >> 2) & 3); }
 
 // Item i of the split of W: a piece of 8 k of one output row.
 __device__ __forceinline__ void split_w(const LinParams& P, uint16_t* Wp, int32_t a_pad, int64_t i) {
@@ -113,14 +113,16 @@ __device__ __forceinline__ void split_w(const LinParams& P, uint16_t* Wp, int32_
 // draws rows [q rc, q rc + rc) of one pair after one jump to the group's start
 // and stores them for both members.  Bound by the draw's vector instructions
 // (about 106 per normal): drawing per pair and not per member halves them
-// (4096 members, 2048 rows, rank 1: 42.8 -> FACT_US us).
+// (4096 members, 2048 rows, rank 1: 42.8 -> 37 us).
 // Blocks from fblocks on split W for k_gemm_f32s (Wp, NULL without one): with
 // a_pad output rows, [k chunk of 32][part][output row][32], the 16-byte pieces
 // of a row swizzled as k_gemm_f32s reads them from LDS (slot_of), zero past a
 // and b.  A block takes 256 pieces of 8 k.
-// vec: every group starts 16-byte aligned.
+// vec: every group starts 16-byte aligned.  Fb (rank 1, or NULL): the input-side
+// rows go there as bf16, [member][b], instead of into F.
 __global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_t groups, int32_t pairs,
-                                                 float* __restrict__ F, int32_t vec, int32_t fblocks,
+                                                 float* __restrict__ F, uint16_t* __restrict__ Fb,
+                                                 int32_t vec, int32_t fblocks,
                                                  uint16_t* __restrict__ Wp, int32_t a_pad) {
     __shared__ BmTables t;
     if ((int32_t)blockIdx.x >= fblocks) {
@@ -142,8 +144,15 @@ __global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_
     float* odd = even + (int64_t)rows * r;
     const bool we = m >= 0, wo = m + 1 < P.n;
     const int32_t split = ((P.tmm ? P.a : P.b) - row0) * r;  // normals before the first scaled row
+    const int32_t k0 = row0 - (P.tmm ? P.a : 0);             // input row of normal 0 (rank 1)
     auto one = [&](int32_t i, float v) {
         const float e = i >= split ? v * P.bs : v;
+        if (Fb && k0 + i >= 0 && k0 + i < P.b) {
+            uint16_t* fb = Fb + (int64_t)m * P.b + k0 + i;
+            if (we) fb[0] = f2bf(e);
+            if (wo) fb[P.b] = f2bf(i >= split ? -e : e);
+            return;
+        }
         if (we) even[i] = e;
         if (wo) odd[i] = i >= split ? -e : e;
     };
@@ -163,6 +172,13 @@ __global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_
                 const bool sc = i + u >= split;
                 ep[u] = sc ? v[u] * P.bs : v[u];
                 op[u] = sc ? -ep[u] : ep[u];
+            }
+            if (Fb && k0 + i >= 0 && k0 + i < P.b) {
+                uint16_t* fb = Fb + (int64_t)m * P.b + k0 + i;
+                if (we) *reinterpret_cast<uint2*>(fb) = uint2{pack_bf16x2(e.x, e.y), pack_bf16x2(e.z, e.w)};
+                if (wo)
+                    *reinterpret_cast<uint2*>(fb + P.b) = uint2{pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w)};
+                return;
             }
             if (we) *reinterpret_cast<float4*>(even + i) = e;
             if (wo) *reinterpret_cast<float4*>(odd + i) = o;
@@ -838,7 +854,8 @@ static bool f32_plan(const LinParams& P, bool split, F32Plan* pl) {
 }
 
 // k_factors: the factor rows (rank 0: none) into F, the split of W into Wp (or NULL).
-static int launch_factors_w(LinParams& P, DeviceState* st, hipStream_t s, float* F, uint16_t* Wp) {
+static int launch_factors_w(LinParams& P, DeviceState* st, hipStream_t s, float* F, uint16_t* Wp,
+                            uint16_t* Fb = nullptr) {
     int32_t rc = 1, groups = 0;
     if (P.r > 0) {
         if (!factor_rows(P, &rc, &groups)) return HSES_ERR_UNSUPPORTED;
@@ -853,13 +870,13 @@ static int launch_factors_w(LinParams& P, DeviceState* st, hipStream_t s, float*
     const int64_t blocks = fblocks + (pieces + 255) / 256;
     if (blocks > INT32_MAX) return set_error(HSES_ERR_INVALID_ARG, "too many factor rows");
     hipLaunchKernelGGL(k_factors, dim3((uint32_t)blocks), dim3(256), 0, s, P, rc, groups,
-                       pairs, F, vec, (int32_t)fblocks, Wp, f32_pad(P.a));
+                       pairs, F, Fb, vec, (int32_t)fblocks, Wp, f32_pad(P.a));
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }
 
-int launch_factors(LinParams& P, DeviceState* st, hipStream_t s, float* F) {
-    return P.r < 1 ? HSES_ERR_UNSUPPORTED : launch_factors_w(P, st, s, F, nullptr);
+int launch_factors(LinParams& P, DeviceState* st, hipStream_t s, float* F, uint16_t* Fb) {
+    return P.r < 1 ? HSES_ERR_UNSUPPORTED : launch_factors_w(P, st, s, F, nullptr, Fb);
 }
 
 size_t linear_f32_workspace(int32_t a, int32_t b, int32_t r, int32_t n, int32_t rows_per_member,
