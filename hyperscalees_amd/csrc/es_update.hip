@@ -10,20 +10,25 @@
 // its own signed weight):  g = scale * sum_p sum_c (w_p Ahat_p[:,c]) B_p[:,c]^T,
 // i.e. an (a x b) output with K = pairs * r.
 //
-// Stage 1: a workgroup owns an output tile and a fixed contiguous range of
-// pairs; for each pair it regenerates the tile's rows of Ahat and B into LDS,
-// rank-chunk by rank-chunk (each thread continues its own row's stream), and
-// accumulates with fp32 MFMA.  The partial tile goes to the workspace.
-//   k_es_rows (r >= 32): one thread per generated row.  A tile spans up to 128
-//     rows of a and up to 384 columns of b, with blockDim = the tile's row
-//     count rounded up to a wave, so every generating thread is busy and a
-//     pair's A rows are regenerated once per b tile (C3 fc1: 3 tiles instead
-//     of 7).  Rank chunks are double-buffered in LDS (one barrier per chunk)
-//     and the generation of the next chunk is interleaved with the MFMAs of
-//     the current one.
-//   k_es_partial (r < 32): 128x128 tiles, 256 threads; a k-chunk of 32 columns
-//     holds 32 / r pairs (the pair weight folded into A at generation), so
-//     every thread generates a run of stream rows of one pair per chunk.
+// The normals are drawn once into a record in the workspace, [k = pair * r + rank
+// column][stream row], a bounded part of the pairs at a time (kEsRecBytes), and
+// contracted from there; drawing inside the contraction repeated every row's
+// draw in each output tile that needs it (8 times at 1024 x 1024).
+//   k_es_draw   one thread per run of stream rows; coalesced over the rows.
+//   r < 32: k_es_gemm  128 x 128 output tiles, split over K chunks of 32.
+//   r >= 32: k_es_rows<.., true>  one thread per stream row.  A tile spans up to
+//     128 rows of a and up to 384 columns of b, with blockDim = the tile's row
+//     count rounded up to a wave.  Rank chunks are double-buffered in LDS (one
+//     barrier per chunk).  hses_es_update_rec runs the same kernel on the
+//     forward's factor record, so the two agree bit for bit.
+// Without a workspace for the record (hses_es_update_noalloc's fixed scratch, or
+// r >= 32 with a split's record past the bound) the contraction draws:
+//   k_es_partial (r < 32): 128x128 tiles, fp32 MFMA, a k-chunk of 32 columns holds
+//     32 / r pairs, so every thread generates a run of stream rows per chunk.
+//   k_es_rows<.., false>: the generation of the next rank chunk is interleaved with
+//     the MFMAs of the current one.
+// Every workgroup owns an output tile and a fixed contiguous range of pairs (or K
+// chunks); its partial tile goes to the workspace.
 // Stage 2 (k_es_reduce): each output element sums its partials in double in
 // a fixed order (four split ranges, each in four interleaved sums), scales,
 // and stores (or adds).  The split count depends on the problem shape only,
@@ -57,8 +62,10 @@ struct UpdParams {
     const uint32_t* cos_exc;
     const uint64_t* jump;  // row length r
     // k_es_rows<.., true>: the forward's factor record, pair pair_lo + i's raw
-    // normal of stream row j, rank c at rec[(i * r + c) * (a + b) + j]
+    // normal of stream row j, rank c at rec[((i - rec_pair0) * r + c) * (a + b) + j]
     const float* rec;
+    int32_t rec_pair0;  // first pair (from pair_lo) in the record
+    int32_t split0;     // first split of this launch
 };
 
 __host__ __device__ constexpr size_t align_up16(size_t x) { return (x + 15) & ~(size_t)15; }
@@ -198,6 +205,16 @@ __device__ __forceinline__ void split_f16x4(const float (&x)[4], uint2* hi, uint
     *lo = __builtin_bit_cast(uint2, l);
 }
 
+// 2^e, the operand scale for terms of at most `top`.
+__device__ __forceinline__ float scale_exponent(float top, int* e) {
+    *e = 0;
+    if (top > 0.0f && isfinite(top)) {
+        frexpf(32768.0f / top, e);
+        *e = min(max(*e - 1, -100), 100);  // 2^e <= 2^15 / top
+    }
+    return ldexpf(1.0f, *e);
+}
+
 // Operand scale S (a power of two) of k_es_rows, and 1/S for k_es_reduce.
 // The A operand is S * (w_p * Ahat): |Ahat| <= base_sigma * 6.44 (the largest
 // Box-Muller radius, u1 >= 2^-24) and |w_p| <= 2 max|f|, so S puts the largest
@@ -215,13 +232,8 @@ __global__ __launch_bounds__(1024) void k_es_scale(const float* __restrict__ f, 
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        const float top = 2.0f * red[0] * fabsf(bs) * 6.5f;  // bound on |w_p * Ahat|
-        int e = 0;
-        if (top > 0.0f && isfinite(top)) {
-            frexpf(32768.0f / top, &e);
-            e = min(max(e - 1, -100), 100);  // 2^e <= 2^15 / top
-        }
-        out[0] = ldexpf(1.0f, e);
+        int e;
+        out[0] = scale_exponent(2.0f * red[0] * fabsf(bs) * 6.5f, &e);  // bound on |w_p * Ahat|
         out[1] = ldexpf(1.0f, -e);
     }
 }
@@ -252,7 +264,7 @@ __global__ __launch_bounds__(R_MAXT) void k_es_rows(UpdParams P, RowTiles G) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nw = blockDim.x >> 6;
     const int32_t q0 = G.q_base + blockIdx.x * bt, o0 = G.o_base + blockIdx.y * at;
-    const int32_t s = blockIdx.z;
+    const int32_t s = P.split0 + blockIdx.z;
     const int32_t p_begin = P.pair_lo + split_begin(P.n_pairs, P.splits, s);
     const int32_t p_end = P.pair_lo + split_begin(P.n_pairs, P.splits, s + 1);
     const int32_t r = P.r;
@@ -343,7 +355,7 @@ __global__ __launch_bounds__(R_MAXT) void k_es_rows(UpdParams P, RowTiles G) {
     float pv[U_CW], pw[U_CW];
     const int64_t rstride = (int64_t)P.a + P.b;  // floats between a row's ranks
     auto load_item = [&](float (&pr)[U_CW], int32_t p, int32_t ch) {
-        const float* src = P.rec + ((int64_t)(p - P.pair_lo) * r + ch * U_CW) * rstride + srow;
+        const float* src = P.rec + ((int64_t)(p - P.pair_lo - P.rec_pair0) * r + ch * U_CW) * rstride + srow;
         const int32_t cn = min(U_CW, r - ch * U_CW);
 #pragma unroll
         for (int c = 0; c < U_CW; ++c)
@@ -477,6 +489,197 @@ __global__ __launch_bounds__(R_MAXT) void k_es_rows(UpdParams P, RowTiles G) {
     }
 }
 
+// ---- the record --------------------------------------------------------------
+
+// The normals of pairs [pair0, pair0 + pairs) (counted from P.pair_lo) into rec:
+// [(pair - pair0) * r + c][stream row].  A thread draws rc consecutive rows of one
+// pair after one jump.  WEIGHT (k_es_gemm): the A rows (stream rows b ..) are
+// stored as (v * bs) * w with the pair's weight w, the reference's fp32 products,
+// and the last block writes {S, 1/S} (k_es_scale) to scale.  Bound by the draw's
+// vector instructions (106 per normal, 300 G normals/s).
+template <bool WEIGHT>
+__global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int32_t pairs, int32_t groups,
+                                                 float* __restrict__ rec, int32_t vec,
+                                                 float* __restrict__ scale) {
+    __shared__ BmTables t;
+    if (WEIGHT && blockIdx.x == gridDim.x - 1) {
+        __shared__ float red[4];
+        float m = 0.0f;
+        for (int32_t i = threadIdx.x; i < P.n; i += 256) m = fmaxf(m, fabsf(P.f[i]));
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+            int e;
+            scale[0] = scale_exponent(2.0f * m * fabsf(P.bs) * 6.5f, &e);  // bound on |w_p * Ahat|
+            scale[1] = ldexpf(1.0f, -e);
+        }
+        return;
+    }
+    load_bm_tables(&t, P.tables);
+    __syncthreads();
+    const int64_t item = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (item >= (int64_t)pairs * groups) return;
+    const int32_t lp = (int32_t)(item / groups), q = (int32_t)(item - (int64_t)lp * groups);
+    const int32_t r = P.r, rows = P.a + P.b, row0 = q * P.rc;
+    const int32_t p = P.pair_lo + pair0 + lp;
+    int32_t te, tt;
+    float sg;
+    epoch_thread_sign(P.epoch, 2 * p, P.nreuse, &te, &tt, &sg);
+    uint64_t st = row_start_state(noise_seed(P.key, te, tt), q, P.jump);
+    const NoiseCtx ctx{&t, P.log_exc, P.cos_exc};
+    float w = 0.0f;
+    if constexpr (WEIGHT) {
+        const int32_t me = 2 * p - P.tid_lo, mo = me + 1;
+        w = ((me >= 0 && me < P.n) ? P.f[me] : 0.0f) - ((mo >= 0 && mo < P.n) ? P.f[mo] : 0.0f);
+    }
+    float* dst = rec + (int64_t)lp * r * rows + row0;
+    const int32_t count = min(P.rc, rows - row0) * r;
+    int32_t row = 0, c = 0;  // of the next normal (normals come in stream order)
+    auto one = [&](int32_t, float v) {
+        if constexpr (WEIGHT) v = row0 + row >= P.b ? (v * P.bs) * w : v;
+        dst[(int64_t)c * rows + row] = v;
+        if (++c == r) c = 0, ++row;
+    };
+    bm_run2<4>(
+        st, count, ctx,
+        [&](int32_t i, const float* v) {
+            if (vec) {  // rank 1, whole aligned groups on one side
+                const bool aside = WEIGHT && row0 + i >= P.b;
+                float4 x{v[0], v[1], v[2], v[3]};
+                if (aside) x = float4{(v[0] * P.bs) * w, (v[1] * P.bs) * w, (v[2] * P.bs) * w, (v[3] * P.bs) * w};
+                *reinterpret_cast<float4*>(dst + i) = x;
+                row += 4;
+                return;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) one(i + u, v[u]);
+        },
+        one);
+}
+
+// ---- k_es_gemm ------------------------------------------------------------------
+// partial[s] = sum over the split's k of (S A[o, k]) B[q, k] from k_es_draw's record
+// (k = pair * r + rank column from the record's first pair).  128 x 128 tiles, four
+// waves of 64 x 64 on fp16 MFMA 32x32x16 with split operands as in k_es_rows
+// (x = xh + xl; hi hi + hi lo + lo hi).  Thread t stages stream row t of the tile
+// (A rows, then B rows): its 32 k of a chunk are 32 loads, each coalesced over the
+// rows, one chunk ahead (two chunks ahead in two register sets: 62 -> 65 us); the LDS rows (hi 64 B, lo 64 B, pitch 144 B: a 16-byte
+// read's 16 lanes fall on distinct banks) are double-buffered, one barrier per
+// chunk.  1024 x 1024 at rank 1 and 4096 members (K 2048, 8 splits of 8 chunks): 30
+// us of the call's 62 (draw 27, reduction 11; 202 us drawing in the contraction),
+// the conversions to operand halves about as long as the MFMAs.
+struct GemmSplit {
+    int64_t k_all, rec_k0;  // k of the whole call, and of the record's first column
+    int32_t chunks;         // K chunks of the whole call
+};
+constexpr int E_HP = 72;  // LDS row pitch (halves)
+
+typedef float f32x16e __attribute__((ext_vector_type(16)));
+
+__global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    uint16_t* lds = reinterpret_cast<uint16_t*>(smem);  // [2][256][E_HP]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lc = lane & 31, kh = lane >> 5;
+    const int32_t q0 = blockIdx.x * U_TB, o0 = blockIdx.y * U_TA;
+    const int32_t bt = min(U_TB, P.b - q0), at = min(U_TA, P.a - o0);
+    const int32_t s = P.split0 + blockIdx.z;
+    // K chunks [c0, c1) of this split, as k (the last chunk of all may be short)
+    const int32_t c0 = split_begin(G.chunks, P.splits, s), c1 = split_begin(G.chunks, P.splits, s + 1);
+    const float S = P.scale[0];
+    const bool is_a = tid < 128;
+    const int32_t lr = is_a ? tid : tid - 128;
+    const bool on = lr < (is_a ? at : bt);
+    const float sc = is_a ? S : 1.0f;
+    const int64_t rows = (int64_t)P.a + P.b;
+    const float* src = P.rec + (on ? (is_a ? P.b + o0 + lr : q0 + lr) : 0);
+    float pv[U_CW];
+    auto load = [&](int32_t ch) {
+        const int64_t k0 = (int64_t)ch * U_CW - G.rec_k0;
+        const int32_t cn = (int32_t)min<int64_t>(U_CW, G.k_all - (int64_t)ch * U_CW);
+#pragma unroll
+        for (int c = 0; c < U_CW; ++c) pv[c] = (on && c < cn) ? src[(k0 + c) * rows] : 0.0f;
+    };
+    auto store = [&](int buf) {
+        uint16_t* dst = lds + (buf * 256 + tid) * E_HP;
+#pragma unroll
+        for (int c = 0; c < U_CW; c += 8) {
+            uint2 h[2], l[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = pv[c + 4 * u + e] * sc;
+                split_f16x4(x, &h[u], &l[u]);
+            }
+            *reinterpret_cast<uint4*>(dst + c) = uint4{h[0].x, h[0].y, h[1].x, h[1].y};
+            *reinterpret_cast<uint4*>(dst + U_CW + c) = uint4{l[0].x, l[0].y, l[1].x, l[1].y};
+        }
+    };
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    f32x16e acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    auto mfma = [](const uint4& a, const uint4& b, f32x16e c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b),
+                                                      c, 0, 0, 0);
+    };
+    if (c0 < c1) load(c0);
+    for (int32_t ch = c0; ch < c1; ++ch) {
+        const int buf = (ch - c0) & 1;
+        store(buf);
+        __syncthreads();  // also: every wave is past chunk ch - 1, whose buffer ch + 1 takes
+        if (ch + 1 < c1) load(ch + 1);
+        const uint16_t* A = lds + buf * 256 * E_HP;
+        const uint16_t* B = A + 128 * E_HP;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int off = 16 * ks + 8 * kh;
+            uint4 ah[2], al[2], bh[2], bl[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                ah[i] = *reinterpret_cast<const uint4*>(A + (wm + 32 * i + lc) * E_HP + off);
+                al[i] = *reinterpret_cast<const uint4*>(A + (wm + 32 * i + lc) * E_HP + U_CW + off);
+                bh[i] = *reinterpret_cast<const uint4*>(B + (wn + 32 * i + lc) * E_HP + off);
+                bl[i] = *reinterpret_cast<const uint4*>(B + (wn + 32 * i + lc) * E_HP + U_CW + off);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma(ah[i], bh[j], acc[i][j]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma(ah[i], bl[j], acc[i][j]);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = mfma(al[i], bh[j], acc[i][j]);
+        }
+    }
+    // element e of lane l: row 8 (e / 4) + 4 kh + e % 4 of the 32-row tile, column lc
+    float* out = P.work + (size_t)s * P.a * P.b;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int col = wn + 32 * j + lc;
+            if (col >= bt) continue;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = wm + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
+                if (row < at) out[(size_t)(o0 + row) * P.b + q0 + col] = acc[i][j][e];
+            }
+        }
+}
+
 // 64 output elements per 256-thread block: wave w sums the partials of splits
 // [w * splits / 4, (w + 1) * splits / 4) of element 64 * block + lane with four
 // interleaved double accumulators, and the four waves' sums are added in wave
@@ -571,6 +774,53 @@ static void pair_range(int32_t tid_lo, int32_t n, int32_t* lo, int32_t* cnt) {
     *cnt = (tid_lo + n - 1) / 2 - *lo + 1;
 }
 
+// How one call runs: the record of `per` consecutive splits at a time (draw), or
+// drawing inside the contraction.  Shape only.
+struct EsPlan {
+    bool draw;
+    int32_t splits, chunks, per;
+    size_t part_bytes, rec_bytes;
+};
+
+// Bound on the record.  Each part of the pairs is a launch of its own that has to
+// fill the card: 1501 pairs x 700 rows at rank 48 (201 MB) took 603 us in two parts
+// of at most 128 MB and 388 us in one (957 drawing in the contraction).
+constexpr size_t kEsRecBytes = 512u << 20;
+
+static EsPlan es_plan(int32_t a, int32_t b, int32_t rank, int32_t n_pairs, bool draw) {
+    EsPlan pl{};
+    const int64_t row_bytes = ((int64_t)a + b) * 4, K = (int64_t)n_pairs * rank;
+    const bool rows_k = use_rows_kernel(rank);
+    int64_t pairs = 0;  // of `per` splits, at most
+    if (rows_k) {
+        pl.splits = rows_splits(a, b, n_pairs);
+        const int64_t each = (n_pairs + pl.splits - 1) / pl.splits;
+        const int64_t bytes = each * rank * row_bytes;
+        pl.draw = draw && bytes <= (int64_t)kEsRecBytes;
+        pl.per = (int32_t)std::min<int64_t>(pl.splits, std::max<int64_t>(1, (int64_t)kEsRecBytes / bytes));
+        pairs = each * pl.per;
+    } else if (!draw) {
+        pl.splits = es_splits(a, b, n_pairs, rank);
+    } else {
+        // k_es_gemm: two workgroups per CU, at least two K chunks each, and no
+        // more k per split than the record's bound
+        pl.draw = true;
+        const int64_t tiles = (int64_t)((a + U_TA - 1) / U_TA) * ((b + U_TB - 1) / U_TB);
+        const int64_t chunks = (K + U_CW - 1) / U_CW;
+        int64_t sp = std::max<int64_t>(1, std::min<int64_t>(512 / tiles, chunks / 2));
+        sp = std::max(sp, (K * row_bytes + (int64_t)kEsRecBytes - 1) / (int64_t)kEsRecBytes);
+        pl.splits = (int32_t)std::min(sp, chunks);
+        pl.chunks = (int32_t)chunks;
+        const int64_t each = (chunks + pl.splits - 1) / pl.splits * U_CW;  // k per split
+        const int64_t room = (int64_t)kEsRecBytes / row_bytes - 2 * rank;
+        pl.per = (int32_t)std::min<int64_t>(pl.splits, std::max<int64_t>(1, room / each));
+        pairs = pl.per * each / rank + 2;
+    }
+    pl.part_bytes = align_up16((size_t)pl.splits * a * b * sizeof(float));
+    pl.rec_bytes = pl.draw ? (size_t)(std::min<int64_t>(pairs, n_pairs) * rank * row_bytes) : 0;
+    return pl;
+}
+
 }  // namespace hses
 
 using namespace hses;
@@ -579,49 +829,47 @@ extern "C" size_t hses_es_update_workspace(int32_t a, int32_t b, int32_t rank, i
     if (a <= 0 || b <= 0 || n <= 0 || rank <= 0) return 0;
     int32_t lo, cnt;
     pair_range(0, n, &lo, &cnt);
-    // tid_lo parity can add one pair; size for the larger count.
-    const int32_t splits = use_rows_kernel(rank) ? rows_splits(a, b, cnt + 1) : es_splits(a, b, cnt + 1, rank);
-    return align_up16((size_t)splits * a * b * sizeof(float)) + 16;  // partials, then {S, 1/S}
+    // tid_lo parity can add one pair; size for either count.  Partials, {S, 1/S}, record.
+    auto bytes = [&](int32_t pairs) {
+        const EsPlan pl = es_plan(a, b, rank, pairs, true);
+        return pl.part_bytes + 16 + pl.rec_bytes;
+    };
+    return std::max(bytes(cnt), bytes(cnt + 1));
 }
 
-// The ES update into a caller's partials buffer: d_work of work_bytes, or,
-// with scratch_cap > 0, at most scratch_cap bytes of it (the split count is
-// lowered until the partials fit).
+// The ES update into a caller's workspace: d_work of work_bytes, or, with
+// scratch_cap > 0, at most scratch_cap bytes of partials in it and no record (the
+// split count is lowered until the partials fit).  rec: the forward's record.
 static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t key, int32_t rank,
                           float sigma, int32_t epoch, int32_t noise_reuse, int32_t a, int32_t b,
                           float scale, int32_t accumulate, float* d_grad, void* d_work,
                           size_t work_bytes, size_t scratch_cap, DeviceState* st,
                           hipStream_t s, const float* rec = nullptr) {
-    UpdParams P{};
-    int32_t pair_lo, n_pairs;
-    pair_range(tid_lo, n, &pair_lo, &n_pairs);
-    const bool empty = n == 0 || rank == 0 || sigma == 0.0f;
-    const bool rows_k = use_rows_kernel(rank);
-    P.splits = empty ? 1 : rows_k ? rows_splits(a, b, n_pairs) : es_splits(a, b, n_pairs, rank);
-    const size_t elems = (size_t)a * b;
-    if (scratch_cap) {
-        const size_t fit = (scratch_cap - 16) / (elems * sizeof(float));
-        if (fit < 1)
-            return set_error(HSES_ERR_INVALID_ARG, "a * b exceeds the fixed scratch of the "
-                                                   "allocation-free ES update");
-        P.splits = (int32_t)std::min<size_t>((size_t)P.splits, fit);
-    }
-    const size_t part_bytes = align_up16((size_t)P.splits * elems * sizeof(float));
-    const size_t need = part_bytes + 16;
-    if (!empty) {
-        HSES_REQUIRE(d_f, "fitness is NULL");
-        HSES_REQUIRE(d_work && work_bytes >= need, "workspace too small");
-    }
-    int rc;
-    if (empty) {
+    const int64_t len = (int64_t)a * b;
+    if (n == 0 || rank == 0 || sigma == 0.0f) {
         if (!accumulate) {
-            const int64_t len = (int64_t)a * b;
             hipLaunchKernelGGL(k_zero, dim3((uint32_t)((len + 255) / 256)), dim3(256), 0, s,
                                d_grad, len);
             HSES_CHECK_HIP(hipGetLastError());
         }
         return HSES_OK;
     }
+    UpdParams P{};
+    int32_t pair_lo, n_pairs;
+    pair_range(tid_lo, n, &pair_lo, &n_pairs);
+    const bool rows_k = use_rows_kernel(rank);
+    EsPlan pl = es_plan(a, b, rank, n_pairs, !rec && !scratch_cap);
+    if (scratch_cap) {
+        const size_t fit = (scratch_cap - 16) / ((size_t)len * sizeof(float));
+        if (fit < 1)
+            return set_error(HSES_ERR_INVALID_ARG, "a * b exceeds the fixed scratch of the "
+                                                   "allocation-free ES update");
+        pl.splits = (int32_t)std::min<size_t>((size_t)pl.splits, fit);
+        pl.part_bytes = align_up16((size_t)pl.splits * len * sizeof(float));
+    }
+    HSES_REQUIRE(d_f, "fitness is NULL");
+    HSES_REQUIRE(d_work && work_bytes >= pl.part_bytes + 16 + pl.rec_bytes, "workspace too small");
+    P.splits = pl.splits;
     P.f = d_f;
     P.n = n;
     P.tid_lo = tid_lo;
@@ -636,12 +884,13 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
     P.n_pairs = n_pairs;
     P.rc = rank >= U_CW ? 1 : std::max(1, U_CW / rank);
     P.work = static_cast<float*>(d_work);
-    float* d_scale = reinterpret_cast<float*>(static_cast<char*>(d_work) + part_bytes);
+    float* d_scale = reinterpret_cast<float*>(static_cast<char*>(d_work) + pl.part_bytes);
     P.scale = d_scale;
     P.tables = st->d_tables;
     P.log_exc = st->d_log_exc;
     P.cos_exc = st->d_cos_exc;
     P.rec = rec;
+    int rc;
     if (rec) {
         HSES_REQUIRE(rows_k, "the factor record update needs rank >= 32");
     } else {
@@ -651,7 +900,10 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
     if (rows_k) {
         hipLaunchKernelGGL(k_es_scale, dim3(1), dim3(1024), 0, s, P.f, n, P.bs, d_scale);
         HSES_CHECK_HIP(hipGetLastError());
-        // One launch per (a-tile, full / remainder b-tile) group.
+    }
+    // k_es_rows of `splits` splits from P.split0: one launch per (a-tile, full /
+    // remainder b-tile) group.
+    auto launch_rows = [&](int32_t splits, bool from_rec) -> int {
         for (int32_t o0 = 0; o0 < a; o0 += 128) {
             const int32_t at = std::min(128, a - o0), btm = rows_bt_max(at);
             const int32_t nfull = b / btm, rem = b % btm;
@@ -660,7 +912,7 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
                 if (cnt == 0) continue;
                 RowTiles G{at, bt, o0, g == 0 ? 0 : nfull * btm};
                 const int32_t threads = (at + bt + 63) / 64 * 64;
-                const size_t lds = (rec ? 0 : align_up16(sizeof(BmTables))) +
+                const size_t lds = (from_rec ? 0 : align_up16(sizeof(BmTables))) +
                                    (size_t)2 * (at + bt + 1) * R_HP * 2;
                 const int32_t nw = threads / 64, nct = (bt + 15) / 16;
                 const int32_t ct = (nct + nw - 1) / nw;
@@ -668,7 +920,7 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
                     if (lds > 64 * 1024)
                         HSES_CHECK_HIP(hipFuncSetAttribute(
                             (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                    hipLaunchKernelGGL(kern, dim3(cnt, 1, P.splits), dim3(threads), lds, s, P, G);
+                    hipLaunchKernelGGL(kern, dim3(cnt, 1, splits), dim3(threads), lds, s, P, G);
                     HSES_CHECK_HIP(hipGetLastError());
                     return HSES_OK;
                 };
@@ -680,18 +932,74 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
                     return ct == 1 ? launch(k_es_rows<8, 1, RC>)
                            : ct == 2 ? launch(k_es_rows<8, 2, RC>) : launch(k_es_rows<8, 3, RC>);
                 };
-                const int lrc = rec ? by_src(std::true_type{}) : by_src(std::false_type{});
+                const int lrc = from_rec ? by_src(std::true_type{}) : by_src(std::false_type{});
                 if (lrc) return lrc;
             }
         }
+        return HSES_OK;
+    };
+    if (pl.draw) {
+        float* d_rec = d_scale + 4;
+        P.rec = d_rec;
+        // rows per drawing thread: up to 16 normals, fewer while that leaves under
+        // 128k threads (as the forward's factor draw)
+        const int32_t rows = a + b;
+        const int64_t K = (int64_t)n_pairs * rank;
+        for (int32_t s0 = 0; s0 < pl.splits; s0 += pl.per) {
+            const int32_t cnt = std::min(pl.per, pl.splits - s0);
+            int32_t p0, p1;  // pairs of these splits
+            if (rows_k) {
+                p0 = split_begin(n_pairs, pl.splits, s0);
+                p1 = split_begin(n_pairs, pl.splits, s0 + cnt);
+            } else {
+                const int64_t k0 = (int64_t)split_begin(pl.chunks, pl.splits, s0) * U_CW;
+                const int64_t k1 = std::min(K, (int64_t)split_begin(pl.chunks, pl.splits, s0 + cnt) * U_CW);
+                p0 = (int32_t)(k0 / rank);
+                p1 = (int32_t)((k1 + rank - 1) / rank);
+            }
+            UpdParams D = P;
+            D.rc = std::max(1, 16 / rank);
+            while (D.rc > 1 && (int64_t)(p1 - p0) * ((rows + D.rc - 1) / D.rc) < 131072) D.rc /= 2;
+            const int32_t groups = (rows + D.rc - 1) / D.rc;
+            rc = get_jump_table(st, (int64_t)D.rc * rank, groups, &D.jump);
+            if (rc) return rc;
+            const int64_t blocks = ((int64_t)(p1 - p0) * groups + 255) / 256;
+            HSES_REQUIRE(blocks < INT32_MAX, "too many factor rows");
+            const int32_t vec = rank == 1 && rows % 4 == 0 && b % 4 == 0 && D.rc % 4 == 0 &&
+                                reinterpret_cast<uintptr_t>(d_rec) % 16 == 0;
+            if (rows_k)
+                hipLaunchKernelGGL(k_es_draw<false>, dim3((uint32_t)blocks), dim3(256), 0, s, D, p0,
+                                   p1 - p0, groups, d_rec, vec, d_scale);
+            else  // its last block writes the operand scale
+                hipLaunchKernelGGL(k_es_draw<true>, dim3((uint32_t)blocks + 1), dim3(256), 0, s, D, p0,
+                                   p1 - p0, groups, d_rec, vec, d_scale);
+            HSES_CHECK_HIP(hipGetLastError());
+            P.split0 = s0;
+            if (rows_k) {
+                P.rec_pair0 = p0;
+                rc = launch_rows(cnt, true);
+                if (rc) return rc;
+            } else {
+                constexpr size_t lds = 2 * 256 * E_HP * 2;
+                HSES_CHECK_HIP(hipFuncSetAttribute((const void*)k_es_gemm,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                const dim3 grid((b + U_TB - 1) / U_TB, (a + U_TA - 1) / U_TA, cnt);
+                hipLaunchKernelGGL(k_es_gemm, grid, dim3(256), lds, s, P,
+                                   GemmSplit{K, (int64_t)p0 * rank, pl.chunks});
+                HSES_CHECK_HIP(hipGetLastError());
+            }
+        }
+    } else if (rows_k) {
+        rc = launch_rows(pl.splits, rec != nullptr);
+        if (rc) return rc;
     } else {
         dim3 grid((b + U_TB - 1) / U_TB, (a + U_TA - 1) / U_TA, P.splits);
         hipLaunchKernelGGL(k_es_partial, grid, dim3(U_THREADS), 0, s, P);
         HSES_CHECK_HIP(hipGetLastError());
     }
-    const int64_t len = (int64_t)a * b;
+    const bool scaled = rows_k || pl.draw;  // the partials are S times the sums
     hipLaunchKernelGGL(k_es_reduce, dim3((uint32_t)((len + 63) / 64)), dim3(256), 0, s, P.work,
-                       P.splits, len, scale, rows_k ? d_scale + 1 : nullptr, accumulate, d_grad);
+                       P.splits, len, scale, scaled ? d_scale + 1 : nullptr, accumulate, d_grad);
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }
@@ -711,15 +1019,12 @@ extern "C" int hses_es_update(const float* d_f, int32_t n, int32_t tid_lo, uint6
                               void* d_work, size_t work_bytes, void* stream) {
     int rc = es_update_check(n, tid_lo, rank, noise_reuse, a, b, d_grad);
     if (rc) return rc;
-    const bool empty = n == 0 || rank == 0 || sigma == 0.0f;
-    if (!empty) {
+    if (n != 0 && rank != 0 && sigma != 0.0f) {
         int32_t lo, cnt;
         pair_range(tid_lo, n, &lo, &cnt);
-        const int32_t splits = use_rows_kernel(rank) ? rows_splits(a, b, cnt)
-                                                     : es_splits(a, b, cnt, rank);
+        const EsPlan pl = es_plan(a, b, rank, cnt, true);
         HSES_REQUIRE(d_f, "fitness is NULL");
-        HSES_REQUIRE(d_work && work_bytes >= align_up16((size_t)splits * a * b * sizeof(float)) + 16,
-                     "workspace too small");
+        HSES_REQUIRE(d_work && work_bytes >= pl.part_bytes + 16 + pl.rec_bytes, "workspace too small");
     }
     DeviceState* st;
     rc = get_state(&st);

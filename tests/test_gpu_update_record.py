@@ -1,0 +1,55 @@
+"""The ES update's own record (hses_es_update: k_es_draw, then k_es_gemm below
+rank 32 or k_es_rows) against the oracle's double-accumulated sum, at the edges of
+its tiles, K chunks and pair ranges.
+
+Bound: the split operands leave out less than 2^-20 of a term and each of the K
+fp32 sums rounds by half an ulp of a partial sum: 2^-20 + 2^-24 sqrt(K) of the sum
+of |terms|, which by the normals' independence is below sqrt(K) times the
+gradient's root mean square per element."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from tests.test_gpu_update import gpu_grad, oracle_grad
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("a,b,r,n,tid_lo", [
+    (1, 1, 1, 2, 0),            # one pair, one output
+    (1, 5, 1, 1, 3),            # one unpaired member
+    (129, 127, 1, 33, 1),       # one row past a tile; K chunks that pairs do not fill
+    (128, 128, 1, 4096, 0),     # aligned groups of four (wide stores), 32 splits
+    (130, 386, 3, 301, 5),      # a chunk ends inside a pair
+    (64, 64, 8, 1024, 0),
+    (300, 20, 31, 77, 2),       # largest rank of the chunked form
+    (200, 500, 48, 301, 0),     # k_es_rows from the record, several tiles
+    (10, 33, 32, 40, 1),
+])
+def test_own_record(hses_gpu, a, b, r, n, tid_lo):
+    fit = np.random.default_rng(a + b + r).standard_normal(n).astype(np.float32)
+    ref = oracle_grad(0.02, r, fit, a, b, tid_lo)
+    g = gpu_grad(hses_gpu, 0.02, r, fit, a, b, np.float32(1.0), tid_lo).cpu().numpy()
+    K = (n + 1) // 2 * r + r
+    tol = (2.0 ** -20 + 2.0 ** -24 * math.sqrt(K)) * math.sqrt(K) * max(np.sqrt((ref ** 2).mean()),
+                                                                        np.abs(ref).max() / 8)
+    assert np.abs(g - ref).max() <= tol, (np.abs(g - ref).max(), tol)
+    # a second call into the same workspace, and one that adds
+    g2 = gpu_grad(hses_gpu, 0.02, r, fit, a, b, np.float32(1.0), tid_lo)
+    assert np.array_equal(g, g2.cpu().numpy())
+    g3 = gpu_grad(hses_gpu, 0.02, r, fit, a, b, np.float32(1.0), tid_lo, out=g2.clone(), accumulate=True)
+    assert torch.equal(g3, g2 + g2)
+
+
+def test_zero_fitness_and_scale_range(hses_gpu):
+    """All-zero fitness gives zeros; fitness at either end of fp32 keeps the
+    relative bar (the operand scale follows max |f|)."""
+    fit = np.zeros(64, np.float32)
+    assert not gpu_grad(hses_gpu, 0.1, 2, fit, 40, 50, np.float32(1.0)).any()
+    base = np.random.default_rng(1).standard_normal(64).astype(np.float32)
+    ref = oracle_grad(0.1, 2, base, 40, 50)
+    for e in (-60, 60):
+        g = gpu_grad(hses_gpu, 0.1, 2, base * np.float32(2.0 ** e), 40, 50, np.float32(2.0 ** -e))
+        assert np.abs(g.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
