@@ -418,6 +418,10 @@ static int run_linear(LinParams& P, DeviceState* st, float* d_y, int64_t y_strid
     int rc = y_fmt == HSES_FMT_F32 ? launch_linear_pair(P, st, s, d_work, work_bytes)
                                    : HSES_ERR_UNSUPPORTED;
     if (rc == HSES_ERR_UNSUPPORTED) {
+        // a few rows in one launch; bf16 outputs where the wide-output kernel offers them
+        rc = y_fmt == HSES_FMT_F32 || linear_wide_applies(P) ? launch_linear_few(P, st, s, act, y_fmt)
+                                                            : HSES_ERR_UNSUPPORTED;
+        if (rc != HSES_ERR_UNSUPPORTED) return rc;  // activation fused
         rc = launch_linear_bf16(P, st, s, d_work, work_bytes, act, y_fmt);
         if (rc != HSES_ERR_UNSUPPORTED) return rc;  // activation fused
         rc = launch_linear_wide(P, st, s, d_work, work_bytes, act, y_fmt);

@@ -214,6 +214,10 @@ size_t linear_wide_workspace(int32_t a, int32_t b, int32_t r, int32_t n, int32_t
                              int32_t n_time, int32_t math);
 int launch_linear_wide(LinParams& P, DeviceState* st, hipStream_t s, void* work, size_t work_bytes,
                        int32_t act, int32_t y_fmt = HSES_FMT_F32);
+// Whether its shape rule takes the call (the workspace and LDS aside).
+bool linear_wide_applies(const LinParams& P);
+// At most 64 rows, small ranks: one launch (linear_few.hip).
+int launch_linear_few(LinParams& P, DeviceState* st, hipStream_t s, int32_t act, int32_t y_fmt);
 // W (a, b) fp32 -> (a, kp) bf16, zero columns [b, kp); tmm: W is stored (b, a).
 void launch_w_to_bf16(const float* W, int32_t a, int32_t b, int32_t kp, int32_t tmm, uint16_t* out,
                       hipStream_t s);

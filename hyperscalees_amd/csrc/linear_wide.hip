@@ -311,21 +311,25 @@ size_t linear_wide_workspace(int32_t a, int32_t b, int32_t r, int32_t n, int32_t
     return align16((size_t)a * wide_kp(b) * 2);
 }
 
-int launch_linear_wide(LinParams& P, DeviceState* st, hipStream_t s, void* work, size_t work_bytes,
-                       int32_t act, int32_t y_fmt) {
-    if (P.math != HSES_MATH_BF16) return HSES_ERR_UNSUPPORTED;
+bool linear_wide_applies(const LinParams& P) {
+    if (P.math != HSES_MATH_BF16) return false;
     if (P.x_fmt == HSES_FMT_BITS) {
-        if (reinterpret_cast<uintptr_t>(P.x) % 8) return HSES_ERR_UNSUPPORTED;
+        if (reinterpret_cast<uintptr_t>(P.x) % 8) return false;
     } else {
-        if (P.x_fmt != HSES_FMT_F32 && P.x_fmt != HSES_FMT_BF16) return HSES_ERR_UNSUPPORTED;
+        if (P.x_fmt != HSES_FMT_F32 && P.x_fmt != HSES_FMT_BF16) return false;
         const int32_t vec = P.x_fmt == HSES_FMT_F32 ? 4 : 8;  // elements per 16-byte load
         if (P.b % vec || P.x_stride % vec || (P.n_time > 1 && P.x_plane % vec) ||
             reinterpret_cast<uintptr_t>(P.x) % 16)
-            return HSES_ERR_UNSUPPORTED;
+            return false;
     }
+    return !(P.r > 0 && P.bs != 0.0f) || wide_nm_max(P.R, P.n) * P.r <= KW_NE;
+}
+
+int launch_linear_wide(LinParams& P, DeviceState* st, hipStream_t s, void* work, size_t work_bytes,
+                       int32_t act, int32_t y_fmt) {
+    if (!linear_wide_applies(P)) return HSES_ERR_UNSUPPORTED;
     const bool noisy = P.r > 0 && P.bs != 0.0f;
     const int32_t nm_max = wide_nm_max(P.R, P.n);
-    if (noisy && nm_max * P.r > KW_NE) return HSES_ERR_UNSUPPORTED;
     const int32_t kp = wide_kp(P.b);
     const size_t wbytes = align16((size_t)P.a * kp * 2);
     if (!work || work_bytes < wbytes) return HSES_ERR_UNSUPPORTED;
