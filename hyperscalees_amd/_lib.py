@@ -221,6 +221,18 @@ def check(rc):
     return rc
 
 
+_fns = {}  # name -> the loaded entry point
+
+
+def fn(name):
+    """Entry point `name` of the loaded library."""
+    f = _fns.get(name)
+    if f is None:
+        f = _fns[name] = getattr(load(), name)
+    return f
+
+
 def call(name, *args):
     """Call entry point `name` and raise HsesError on a non-zero status."""
-    return check(getattr(load(), name)(*args))
+    rc = (_fns.get(name) or fn(name))(*args)
+    return rc if rc == HSES_OK else check(rc)

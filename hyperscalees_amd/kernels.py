@@ -16,15 +16,26 @@ _FMT_DTYPE = {FMT_F32: torch.float32, FMT_BF16: torch.bfloat16, FMT_U8: torch.ui
               FMT_BITS: torch.int64}
 
 
+# A call's host time is as long as a small kernel, so the helpers below stay on the
+# cheap side: addresses go to ctypes as ints, and the current stream is read
+# without building a torch.cuda.Stream (about 4 us, twice a call).
 def _p(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def _set_stream(s):
+    """Make torch.cuda.Stream s the current stream (the caller restores it)."""
+    torch._C._cuda_setStream(stream_id=s.stream_id, device_index=s.device_index,
+                             device_type=s.device_type)
 
 
 def _dev(t, dtype, name):
+    if type(t) is torch.Tensor and t.is_cuda and t.dtype is dtype and t.is_contiguous():
+        return t
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise ValueError(f"{name} must be a device tensor")
     if t.dtype != dtype:
@@ -39,12 +50,27 @@ _WORK = {}
 
 def _workspace(nbytes, device):
     """A cached device workspace of at least nbytes (one per device and stream)."""
-    key = (str(device), torch.cuda.current_stream().cuda_stream)
+    key = (device, _stream())
     buf = _WORK.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
         _WORK[key] = buf
     return buf
+
+
+_SIZES = {}
+
+
+def _size(name, *shape):
+    """A size query of the library (a function of the shape alone), asked once per
+    shape; 0 is asked again (a query before hses_init may answer 0)."""
+    key = (name, shape)
+    n = _SIZES.get(key)
+    if not n:
+        if len(_SIZES) > 4096:
+            _SIZES.clear()
+        n = _SIZES[key] = int(_lib.fn(name)(*shape))
+    return n
 
 
 def fmt_width(fmt, width):
@@ -350,8 +376,8 @@ def perturbed_linear(x, W, key, rank, sigma, epoch, noise_reuse, tid_lo, n, rows
     _dev(out, ydt, "out")
     if out.numel() != n_time * M * a:
         raise ValueError("out has the wrong size")
-    wbytes = int(_lib.load().hses_perturbed_linear_workspace(a, b, rank, n, rows_per_member,
-                                                              n_time, math))
+    wbytes = _size("hses_perturbed_linear_workspace", a, b, rank, n, rows_per_member,
+                                                              n_time, math)
     work = _workspace(wbytes, W.device)
     if img is not None:
         if rec is None or act or out_bf16 or math not in (MATH_BF16, MATH_F32X):
@@ -398,8 +424,8 @@ def perturbed_linear_t(x, W, key, rank, sigma, epoch, noise_reuse, tid_lo, n, ro
     _dev(out, ydt, "out")
     if out.numel() != n_time * M * b:
         raise ValueError("out has the wrong size")
-    wbytes = int(_lib.load().hses_perturbed_linear_t_workspace(a, b, rank, n, rows_per_member,
-                                                                n_time, math))
+    wbytes = _size("hses_perturbed_linear_t_workspace", a, b, rank, n, rows_per_member,
+                                                                n_time, math)
     work = _workspace(wbytes, W.device)
     if act or out_bf16:
         _lib.call("hses_perturbed_linear_act", _p(x), x_fmt, units, M * units, n_time, _p(W), a,
@@ -447,8 +473,8 @@ def perturbed_linear_lif(x, W, key, rank, sigma, epoch, noise_reuse, tid_lo, n,
             raise ValueError("rate has the wrong size")
     if math not in (MATH_BF16, MATH_F32X) or (math == MATH_F32X and img is None):
         raise ValueError("the fused forward takes bf16 math, or split math with img")
-    wbytes = int(_lib.load().hses_perturbed_linear_workspace(a, b, rank, n, rows_per_member,
-                                                              n_time, math))
+    wbytes = _size("hses_perturbed_linear_workspace", a, b, rank, n, rows_per_member,
+                                                              n_time, math)
     work = _workspace(wbytes, W.device)
     if time_inner:
         xs, xp, ss, sp = n_time * units, units, n_time * wa, wa
@@ -525,8 +551,8 @@ def perturbed_linear_lif_counts_x(x, W, rank, sigma, tid_lo, n, rows_per_member,
     _dev(counts, torch.int64, "counts")
     if counts.numel() != M * npl * wa:
         raise ValueError("counts has the wrong size")
-    wbytes = int(_lib.load().hses_perturbed_linear_workspace(a, b, rank, n, rows_per_member,
-                                                              n_time, MATH_F32X))
+    wbytes = _size("hses_perturbed_linear_workspace", a, b, rank, n, rows_per_member,
+                                                              n_time, MATH_F32X)
     work = _workspace(wbytes, W.device)
     if time_inner:
         xs, xp = n_time * units, units
@@ -544,8 +570,7 @@ def es_update(fit, tid_lo, key, rank, sigma, epoch, noise_reuse, a, b, scale, ou
     `out` when accumulate is set."""
     _dev(fit, torch.float32, "fit")
     n = fit.numel()
-    lib = _lib.load()
-    wbytes = int(lib.hses_es_update_workspace(a, b, rank, n))
+    wbytes = _size("hses_es_update_workspace", a, b, rank, n)
     if work is None or work.numel() < wbytes:
         work = _workspace(wbytes, fit.device)
     if out is None:
@@ -562,8 +587,7 @@ def es_update_rec(fit, tid_lo, rec, rank, sigma, a, b, scale, out=None, accumula
     (the same result as es_update, without drawing the normals again)."""
     _dev(fit, torch.float32, "fit")
     n = fit.numel()
-    lib = _lib.load()
-    wbytes = int(lib.hses_es_update_workspace(a, b, rank, n))
+    wbytes = _size("hses_es_update_workspace", a, b, rank, n)
     if work is None or work.numel() < wbytes:
         work = _workspace(wbytes, fit.device)
     if out is None:
@@ -686,7 +710,7 @@ def full_update(fit, tid_lo, key, sigma, epoch, noise_reuse, a, b, scale, out=No
     """_simple_full_update of a dense (a, b) parameter: scale * sum_m fit[m] noise_m."""
     _dev(fit, torch.float32, "fit")
     n = fit.numel()
-    wbytes = int(_lib.load().hses_full_update_workspace(a, b, n))
+    wbytes = _size("hses_full_update_workspace", a, b, n)
     work = _workspace(wbytes, fit.device)
     if out is None:
         out = torch.empty((a, b), dtype=torch.float32, device=fit.device)

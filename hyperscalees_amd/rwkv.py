@@ -16,6 +16,7 @@ from . import kernels as K
 from ._lib import ACT_RELU_SQ, ACT_SIGMOID, ACT_TANH, FMT_BF16, FMT_F32, MATH_BF16, MATH_F32
 
 
+FEW_ROWS = 64  # rows (sequences x tokens) of one-launch linears
 _SIDE = {}  # device index -> side streams (default priority)
 
 
@@ -28,9 +29,12 @@ def _side_streams(dev):
 
 def _fan_out(jobs, inputs):
     """Run independent launches round-robin on side streams, joined into the
-    current stream.  `inputs` (made on the current stream) is recorded on the
+    current stream (a few rows: in turn on the current stream, where the joins
+    would cost more than running side by side saves).  `inputs` (made on the current stream) is recorded on the
     side streams and every job's output on the current stream, so the caching
     allocator reuses neither block before the stream that reads it is done."""
+    if inputs.shape[1] * inputs.shape[2] <= FEW_ROWS:
+        return {name: fn() for name, fn in jobs.items()}
     main = torch.cuda.current_stream()
     ready = torch.cuda.Event()
     ready.record(main)
@@ -39,9 +43,12 @@ def _fan_out(jobs, inputs):
         side.wait_event(ready)
         inputs.record_stream(side)
     out = {}
-    for i, (name, fn) in enumerate(jobs.items()):
-        with torch.cuda.stream(sides[i % len(sides)]):
+    try:
+        for i, (name, fn) in enumerate(jobs.items()):
+            K._set_stream(sides[i % len(sides)])
             out[name] = fn()
+    finally:
+        K._set_stream(main)
     for side in sides:
         main.wait_stream(side)
     for t in out.values():

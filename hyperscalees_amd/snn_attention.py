@@ -171,9 +171,12 @@ class SpikingAttentionEs:
         sides = self._side_streams()
         for side in sides:
             side.wait_event(ready)
-        for i, fn in enumerate(calls):
-            with torch.cuda.stream(sides[i % len(sides)]):
+        try:
+            for i, fn in enumerate(calls):
+                K._set_stream(sides[i % len(sides)])
                 fn()
+        finally:
+            K._set_stream(main)
         for side in sides:
             main.wait_stream(side)
 
@@ -185,8 +188,7 @@ class SpikingAttentionEs:
         c = self.cfg
         W = self.P[name]
         a, b = W.shape
-        lib = _lib.load()
-        wbytes = int(lib.hses_perturbed_linear_workspace(a, b, c.rank, n, rpm, n_time, MATH_F32))
+        wbytes = K._size("hses_perturbed_linear_workspace", a, b, c.rank, n, rpm, n_time, MATH_F32)
         work = K._workspace(wbytes, self.dev)
         yp = y.data_ptr() + 4 * y_off
         _lib.call("hses_perturbed_linear", K._p(x), FMT_F32, x_stride, x_plane, n_time, K._p(W),
@@ -301,8 +303,9 @@ class SpikingAttentionEs:
         for side in self._side_streams():
             side.wait_event(ready)
             z.record_stream(side)
-        for i, (name, (a, b), cls) in enumerate(self.leaves):
-            with torch.cuda.stream(self.streams[i % len(self.streams)]):
+        try:
+            for i, (name, (a, b), cls) in enumerate(self.leaves):
+                K._set_stream(self.streams[i % len(self.streams)])
                 if cls == MM:
                     K.es_update(z, 0, self.keys[name], c.rank, c.sigma, epoch, c.noise_reuse, a,
                                 b, scale, out=self.grads[name])
@@ -312,6 +315,8 @@ class SpikingAttentionEs:
                 K.solver_step(c.solver, c.lr, self.P[name], self.grads[name], self.m[name],
                               self.v[name], step_t=self.step_t, beta1=c.beta1, beta2=c.beta2,
                               eps=c.eps, wd=c.weight_decay if c.solver == ADAMW else 0.0)
+        finally:
+            K._set_stream(main)
         for side in self.streams:
             main.wait_stream(side)
         return z
