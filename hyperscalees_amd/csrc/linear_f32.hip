@@ -500,18 +500,27 @@ void k_gemm_f32s(LinParams P, const float* __restrict__ F, const uint16_t* __res
 }
 
 // ---- k_gemm_f32 ------------------------------------------------------------------
+// The epilogue keeps the A_m rows as [member][RK / 4][column][4] in LDS, so that the
+// 32 columns of a 16-byte read fall on distinct banks (as rows of RK they shared
+// eight: 70% of the kernel's LDS cycles at 16 -> 64, rank 8), reads them once when
+// the tile has one member, and takes each row's offset and member from an LDS
+// table (the divisions of 16 rows per lane were most of its vector instructions).
+// Bits do not change: 524288 x 16 -> 64 at rank 8 166 -> 121 us (best 78), 32768 spike
+// rows 256 -> 256 at rank 4 83 -> 65 us.
+//
 // NT 32-column MFMA tiles per wave (BN = 32 NT); four waves of 32 rows.  RK is
 // the rank padded to 1, 4, 8 or 16 (the LDS copies of B_m and A_m rows hold RK
 // values per row, zero past r).
 template <int XFMT, int NT, int RK>
 __global__ __launch_bounds__(KF_THREADS) void k_gemm_f32(LinParams P, const float* __restrict__ F,
-                                                         int32_t bch) {
+                                                         int32_t bch, int32_t nm_max) {
     constexpr int BN = 32 * NT;
     extern __shared__ __align__(16) unsigned char smem[];
     // Two staging buffers, each: 128 x rows, BN W rows (KF_XP floats each), then
     // the chunk's B_m rows of the tile's members ([lm][32][RK]).  After them the
-    // tile's A_m rows ([lm][BN][RK]).  bch (floats of a chunk's B_m rows, 0
-    // without noise) is the host's, which sized the LDS.
+    // tile's A_m rows ([lm][RK / 4][BN][4]) and each row's y offset and member.  bch
+    // (floats of a chunk's B_m rows, 0 without noise) and nm_max (members a tile can
+    // touch) are the host's, which sized the LDS.
     const int32_t bufsz = (KF_BM + BN) * KF_XP + bch;
     float* buf = reinterpret_cast<float*>(smem);
     // one staging buffer when K is a single chunk (b <= 32), else two
@@ -542,12 +551,21 @@ __global__ __launch_bounds__(KF_THREADS) void k_gemm_f32(LinParams P, const floa
     const bool noisy = r > 0;
     const int64_t fpitch = (int64_t)(P.a + b) * r;  // floats of one member's factors
     const float* Fm = F + (int64_t)m_first * fpitch;
+    int64_t* yoffs = reinterpret_cast<int64_t*>(As + (noisy ? nm_max * BN * RK : 0));
+    int32_t* rlm = reinterpret_cast<int32_t*>(yoffs + KF_BM);
+    if (tid < KF_BM) {
+        const bool ok = tid < rows_here;
+        yoffs[tid] = ok ? tr.offset(P, tid, P.y_stride, P.y_plane) + o0 : 0;
+        rlm[tid] = ok ? tr.member(P, tid) : 0;
+    }
 
     // ---- A rows of the tile's members: F rows b + o0 .. b + o0 + ct ------------
+    constexpr int RQ = RK < 4 ? 1 : RK / 4, RC = RK < 4 ? RK : 4;  // [lm][RQ][BN][RC]
     if (noisy) {
         for (int32_t i = tid; i < nm * BN * RK; i += KF_THREADS) {
             const int32_t c = i % RK, o = (i / RK) % BN, lm = i / (RK * BN);
-            As[i] = (c < r && o < ct) ? Fm[lm * fpitch + (int64_t)(b + o0 + o) * r + c] : 0.0f;
+            As[((lm * RQ + c / RC) * BN + o) * RC + c % RC] =
+                (c < r && o < ct) ? Fm[lm * fpitch + (int64_t)(b + o0 + o) * r + c] : 0.0f;
         }
     }
 
@@ -738,26 +756,49 @@ __global__ __launch_bounds__(KF_THREADS) void k_gemm_f32(LinParams P, const floa
     }
     // accumulator element e of lane l: row 8 (e / 4) + 4 kh + e % 4 of the
     // wave's 32, column lc of the tile
+    float ar[NT][RK];
+    auto load_a = [&](int32_t lm) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                const float* p = As + ((lm * RQ + q) * BN + 32 * j + lc) * RC;
+                if constexpr (RC == 4) {
+                    const float4 v = *reinterpret_cast<const float4*>(p);
+                    ar[j][4 * q] = v.x, ar[j][4 * q + 1] = v.y, ar[j][4 * q + 2] = v.z, ar[j][4 * q + 3] = v.w;
+                } else {
+                    ar[j][0] = p[0];
+                }
+            }
+    };
+    if (noisy && nm == 1) load_a(0);
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
         const int32_t row = wave * 32 + 8 * (e >> 2) + 4 * kh + (e & 3);
-        const int64_t L = L0 + row;
-        if (L >= P.total) continue;
-        const int32_t lm = tr.member(P, row);
-        float* yrow = P.y + tr.offset(P, row, P.y_stride, P.y_plane) + o0;
+        if (row >= rows_here) continue;
+        float* yrow = P.y + yoffs[row];
         float xr_[RK];
+        if (noisy) {
+            if (nm > 1) load_a(rlm[row]);
+            if constexpr (RC == 4) {
 #pragma unroll
-        for (int c = 0; c < RK; ++c) xr_[c] = noisy ? XBs[row * RK + c] : 0.0f;
+                for (int q = 0; q < RQ; ++q) {
+                    const float4 v = *reinterpret_cast<const float4*>(XBs + row * RK + 4 * q);
+                    xr_[4 * q] = v.x, xr_[4 * q + 1] = v.y, xr_[4 * q + 2] = v.z, xr_[4 * q + 3] = v.w;
+                }
+            } else {
+                xr_[0] = XBs[row];
+            }
+        }
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             const int32_t col = 32 * j + lc;
             if (col >= ct) continue;
             float yv = acc[j][e];
             if (noisy) {
-                const float* ar = As + ((size_t)lm * BN + col) * RK;
                 float z = 0.0f;
 #pragma unroll
-                for (int c = 0; c < RK; ++c) z = __fadd_rn(z, __fmul_rn(xr_[c], ar[c]));
+                for (int c = 0; c < RK; ++c) z = __fadd_rn(z, __fmul_rn(xr_[c], ar[j][c]));
                 yv = __fadd_rn(yv, z);
             }
             yrow[col] = yv;
@@ -815,7 +856,7 @@ static bool factor_rows(const LinParams& P, int32_t* rc_out, int32_t* groups) {
 // The tiling of one call (shape only).  split: k_gemm_f32s.
 struct F32Plan {
     bool split;
-    int32_t bm, bn, rk, bch;
+    int32_t bm, bn, rk, bch, nm;
     size_t lds, f_bytes, w_bytes;
 };
 
@@ -834,6 +875,7 @@ static bool f32_plan(const LinParams& P, bool split, F32Plan* pl) {
     const size_t bch = r > 0 ? (size_t)nm * KF_BK * pl->rk : 0;
     if (bch > (size_t)(split ? KS_BPT : 8) * KF_THREADS) return false;  // BPT values per thread
     pl->bch = (int32_t)bch;
+    pl->nm = nm;
     const size_t a_lds = r > 0 ? (size_t)nm * pl->bn * pl->rk : 0;
     if (a_lds > KF_AMAX) return false;
     if (split) {
@@ -841,7 +883,7 @@ static bool f32_plan(const LinParams& P, bool split, F32Plan* pl) {
         pl->lds = (parts * pl->bm + 3 * pl->bn) * KF_BK * 2 + bch * 4 + (size_t)pl->bm * 20 + a_lds * 4;
     } else {
         const size_t nbuf = P.b > KF_BK ? 2 : 1;  // staging buffers (k_gemm_f32)
-        pl->lds = (nbuf * ((size_t)(KF_BM + pl->bn) * KF_XP + bch) + a_lds) * 4;
+        pl->lds = (nbuf * ((size_t)(KF_BM + pl->bn) * KF_XP + bch) + a_lds + 3 * KF_BM) * 4;
     }
     pl->w_bytes = split ? f32_w_bytes(P.a, P.b) : 0;
     pl->f_bytes = 0;
@@ -901,10 +943,10 @@ template <int XFMT, int NT>
 static int launch_gemm_rk(const LinParams& P, const F32Plan& pl, hipStream_t s, const float* F,
                           dim3 grid) {
     switch (pl.rk) {
-        case 1: return launch_f32(k_gemm_f32<XFMT, NT, 1>, pl.lds, grid, s, P, F, pl.bch);
-        case 4: return launch_f32(k_gemm_f32<XFMT, NT, 4>, pl.lds, grid, s, P, F, pl.bch);
-        case 8: return launch_f32(k_gemm_f32<XFMT, NT, 8>, pl.lds, grid, s, P, F, pl.bch);
-        default: return launch_f32(k_gemm_f32<XFMT, NT, 16>, pl.lds, grid, s, P, F, pl.bch);
+        case 1: return launch_f32(k_gemm_f32<XFMT, NT, 1>, pl.lds, grid, s, P, F, pl.bch, pl.nm);
+        case 4: return launch_f32(k_gemm_f32<XFMT, NT, 4>, pl.lds, grid, s, P, F, pl.bch, pl.nm);
+        case 8: return launch_f32(k_gemm_f32<XFMT, NT, 8>, pl.lds, grid, s, P, F, pl.bch, pl.nm);
+        default: return launch_f32(k_gemm_f32<XFMT, NT, 16>, pl.lds, grid, s, P, F, pl.bch, pl.nm);
     }
 }
 
