@@ -105,21 +105,42 @@ __global__ __launch_bounds__(kFullThreads) void k_full_partial(
     for (int32_t i = 0; i < cnt; ++i) dst[i] = acc[i][threadIdx.x];
 }
 
-// Stage 2: g[e] = (f32 of the split partials summed in split order) * scale
-// (or added to g with accumulate).
+// Stage 2: g[e] = (f32 of the split partials' sum) * scale (or added to g with
+// accumulate).  A block takes 256 / lanes elements; lane j of an element sums
+// the splits j, j + lanes, ... in order, and the lanes are summed in lane order.
+// With one thread for an element a small leaf's few threads wait for up to 1024
+// loads one after another: 39 us for 1 x 1 at 1024 members (with lanes and full_splits
+// below 165 + 315 -> about 80 us for the nine dense leaves of a spiking attention
+// step, the first of them 64 x 64).
+constexpr int kReduceLanes = 16;
 __global__ __launch_bounds__(256) void k_full_reduce(const double* __restrict__ part, int32_t splits,
-                                                     int64_t E, float scale, int32_t accumulate,
-                                                     float* __restrict__ g) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= E) return;
+                                                     int32_t lanes, int64_t E, float scale,
+                                                     int32_t accumulate, float* __restrict__ g) {
+    __shared__ double sum[256];
+    const int32_t width = 256 / lanes;  // elements of a block
+    const int32_t lane = (int32_t)threadIdx.x / width;
+    const int64_t e = (int64_t)blockIdx.x * width + (int32_t)threadIdx.x % width;
     double s = 0.0;
-    for (int32_t k = 0; k < splits; ++k) s += part[(int64_t)k * E + e];
+    if (e < E) {
+#pragma unroll 8
+        for (int32_t k = lane; k < splits; k += lanes) s += part[(int64_t)k * E + e];
+    }
+    if (lanes > 1) {
+        sum[threadIdx.x] = s;
+        __syncthreads();
+        if (lane == 0)
+            for (int32_t j = 1; j < lanes; ++j) s += sum[j * width + threadIdx.x];
+    }
+    if (e >= E || lane) return;
     const float v = splits ? (float)s * scale : 0.0f;
     g[e] = accumulate ? g[e] + v : v;
 }
 
-static int32_t full_splits(int32_t chunks, int32_t n_pairs) {
-    int64_t s = std::max<int64_t>(1, 4096 / std::max(1, chunks));
+// Splits of the pairs: enough that chunks x splits reach `threads`.  65536 is a wave
+// for each SIMD; callers whose workspace holds only what 4096 threads need get those.
+constexpr int32_t kFullFill = 65536, kFullFillMin = 4096;
+static int32_t full_splits(int32_t chunks, int32_t n_pairs, int32_t threads = kFullFill) {
+    int64_t s = std::max<int64_t>(1, threads / std::max(1, chunks));
     s = std::min<int64_t>(s, std::max(1, n_pairs));
     return (int32_t)std::min<int64_t>(s, 1024);
 }
@@ -231,7 +252,9 @@ extern "C" int hses_full_update(const float* d_f, int32_t n, int32_t tid_lo, uin
     const int64_t chunks = (E + kFullLc - 1) / kFullLc;
     HSES_REQUIRE(chunks <= kJumpMaxRows, "a * b exceeds 32 * 16384 elements");
     const int32_t pair_lo = tid_lo / 2, n_pairs = n ? (tid_lo + n - 1) / 2 - pair_lo + 1 : 0;
-    const int32_t splits = full_splits((int32_t)chunks, n_pairs);
+    int32_t splits = full_splits((int32_t)chunks, n_pairs);
+    if (work_bytes < (size_t)splits * E * sizeof(double))
+        splits = full_splits((int32_t)chunks, n_pairs, kFullFillMin);
     const bool empty = n == 0 || sigma == 0.0f;
     if (!empty) {
         HSES_REQUIRE(d_f, "fitness is NULL");
@@ -242,12 +265,13 @@ extern "C" int hses_full_update(const float* d_f, int32_t n, int32_t tid_lo, uin
     int rc = get_state(&st);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    const uint32_t rblocks = (uint32_t)((E + 255) / 256);
+    const int32_t lanes = splits >= kReduceLanes ? kReduceLanes : 1;
+    const uint32_t rblocks = (uint32_t)((E * lanes + 255) / 256);
     if (empty) {
         if (!accumulate) {
             // zero gradient: reduce over no partials
-            hipLaunchKernelGGL(k_full_reduce, dim3(rblocks), dim3(256), 0, s, nullptr, 0, E, scale,
-                               0, d_grad);
+            hipLaunchKernelGGL(k_full_reduce, dim3(rblocks), dim3(256), 0, s, nullptr, 0, lanes, E,
+                               scale, 0, d_grad);
             HSES_CHECK_HIP(hipGetLastError());
         }
         return HSES_OK;
@@ -262,8 +286,8 @@ extern "C" int hses_full_update(const float* d_f, int32_t n, int32_t tid_lo, uin
                        (int32_t)chunks, pair_lo, n_pairs, splits, part, st->d_tables,
                        st->d_log_exc, st->d_cos_exc, jump);
     HSES_CHECK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_full_reduce, dim3(rblocks), dim3(256), 0, s, part, splits, E, scale,
-                       accumulate, d_grad);
+    hipLaunchKernelGGL(k_full_reduce, dim3(rblocks), dim3(256), 0, s, part, splits, lanes, E,
+                       scale, accumulate, d_grad);
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }
