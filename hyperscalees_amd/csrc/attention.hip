@@ -71,8 +71,12 @@ __global__ __launch_bounds__(256) void k_softplus(const float* __restrict__ x, i
 }
 
 // _rate of the three encoders and their mean plus the position embedding
-// (snn_self_attention_heads.py:33-40, 168-175): one thread per (row, column).
+// (snn_self_attention_heads.py:33-40, 168-175): one thread per row and VEC columns.
 // th_q, th_k, th_v: (n) thresholds; pos: (R, d) shared or (n, R, d).
+// Bound by its 3 T reads: VEC = 4 where every plane's rows are 16-byte aligned, with
+// the three encoders' loads of four steps in flight.
+// 1024 members x 64 tokens x 64, T = 8: 149 -> 92 us (2.9 -> 4.7 TB/s; a copy reaches 4.76).
+template <int VEC>
 __global__ __launch_bounds__(256) void k_sa_encode(const float* __restrict__ cq,
                                                    const float* __restrict__ ck,
                                                    const float* __restrict__ cv, int32_t T,
@@ -82,56 +86,76 @@ __global__ __launch_bounds__(256) void k_sa_encode(const float* __restrict__ cq,
                                                    const float* __restrict__ th_v, float leak,
                                                    const float* __restrict__ pos,
                                                    int32_t pos_per_member, float* __restrict__ X) {
-    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
     const int64_t total = M * d;
     if (e >= total) return;
-    const int64_t row = e / d;
-    const int64_t m = row / R;
-    const float* cs[3] = {cq, ck, cv};
+    const int64_t m = e / ((int64_t)R * d);
+    const float* cs[3] = {cq + e, ck + e, cv + e};
     const float ths[3] = {th_q[m], th_k[m], th_v[m]};
-    float rate[3];
+    float v[3][VEC], cnt[3][VEC];
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const float vth = ths[q];
-        float v = 0.0f, cnt = 0.0f, s;
-        for (int32_t t = 0; t < T; ++t) {
-            v = lif_upd(v, cs[q][(int64_t)t * total + e], leak, vth, &s);
-            cnt = __fadd_rn(cnt, s);
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) v[q][i] = cnt[q][i] = 0.0f;
+#pragma unroll 4
+    for (int32_t t = 0; t < T; ++t) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const vec c = *reinterpret_cast<const vec*>(cs[q] + (int64_t)t * total);
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                float s;
+                v[q][i] = lif_upd(v[q][i], c[i], leak, ths[q], &s);
+                cnt[q][i] = __fadd_rn(cnt[q][i], s);
+            }
         }
-        rate[q] = __fdiv_rn(cnt, (float)T);
     }
-    const int64_t pe = pos_per_member ? e : e % ((int64_t)R * d);
-    X[e] = __fadd_rn(__fdiv_rn(__fadd_rn(__fadd_rn(rate[0], rate[1]), rate[2]), 3.0f), pos[pe]);
+    const vec p = *reinterpret_cast<const vec*>(pos + (pos_per_member ? e : e - m * R * d));
+    vec x;
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        float rate[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) rate[q] = __fdiv_rn(cnt[q][i], (float)T);
+        x[i] = __fadd_rn(__fdiv_rn(__fadd_rn(__fadd_rn(rate[0], rate[1]), rate[2]), 3.0f), p[i]);
+    }
+    *reinterpret_cast<vec*>(X + e) = x;
 }
 
 // One head of multihead_attention_once for one member per workgroup
-// (snn_self_attention_heads.py:54-70 with row_softmax_lif): K, V (and Q) of
-// the member's R tokens staged in LDS (dynamic, sized for R and hd, so that
-// several workgroups share a CU); each wave takes groups of RP = min(4, 64 /
-// hd) query rows.  Per row lane j is key neuron j: h_j = beta (q_i . k_j),
-// normalised by max |h| + 1e-6, n_iter LIF steps with the inhibition g_inh *
-// (sum of counts), p_j = count_j / (sum count + 1e-6) into the wave's LDS
-// rows; then out_i = p @ V for the group's RP rows at once, lane rr * hd + c
-// summing row rr's channel c over j in index order.
+// (snn_self_attention_heads.py:54-70 with row_softmax_lif): Q, K and V of the
+// member's R tokens are staged in LDS; each wave takes groups of NQ query rows.
+// Per row lane j is key neuron j: h_j = beta (q_i . k_j), normalised by max |h| +
+// 1e-6, n_iter LIF steps with the inhibition g_inh * (sum of counts), p_j = count_j /
+// (sum count + 1e-6) into the wave's LDS rows; then out_i = p @ V for 64 / hd rows
+// at once, lane rr * hd + c summing row rr's channel c over j in index order.
+//
+// Bound by vector instructions (bits are the reference's, so mul and add stay apart).
+// The counts' sum is a scalar: it grows by the population count of the spikes' lane
+// mask, so a step needs no reduction over lanes.  Head sizes 8, 16 and 32 have their own
+// instances: a lane's key (hd values) and its V column (64) stay in registers over
+// its wave's rows, and only the uniform q and the p rows are read from LDS, four at a
+// time.  Other sizes read K and V from LDS.
+// 1024 members x 4 heads, 64 tokens, head size 16, 8 steps: 138 -> 94 us (a reduction over
+// lanes in every step, K and V from LDS in every group).
 constexpr int kSaWaves = 4;
-constexpr int kSaMaxR = 64, kSaMaxHd = 64, kSaMaxRP = 4;
-constexpr int kSaPP = kSaMaxR + 1;  // pitch of a wave's p rows (rows on distinct banks)
-static size_t sa_lds_bytes(int32_t R, int32_t hd) {
-    return (3 * (size_t)R * (hd + 1) + (size_t)kSaWaves * kSaMaxRP * kSaPP) * sizeof(float);
-}
+constexpr int kSaMaxR = 64, kSaMaxHd = 64;
+constexpr int kSaPP = kSaMaxR + 4;  // pitch of a wave's p rows (16-byte reads, distinct banks)
+template <int HD, int NQ>
 __global__ __launch_bounds__(kSaWaves * 64) void k_sa_attention(
         const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
-        int32_t ld, int32_t R, int32_t H, int32_t hd, const float* __restrict__ beta,
+        int32_t ld, int32_t R, int32_t H, int32_t hd_, const float* __restrict__ beta,
         const float* __restrict__ vth, float g_inh, float leak, int32_t n_iter,
         float* __restrict__ out) {
-    extern __shared__ float sa_lds[];
-    const int pitch = hd + 1;
-    float* qs = sa_lds;
+    extern __shared__ __align__(16) float sa_lds[];
+    const int hd = HD ? HD : hd_, pitch = HD ? HD + 4 : hd_ + 1;
+    const int m = (int)(blockIdx.x / (uint32_t)H), h = (int)(blockIdx.x % (uint32_t)H);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float* ps = sa_lds + w * (NQ * kSaPP);
+    float* qs = sa_lds + kSaWaves * NQ * kSaPP;
     float* ks = qs + R * pitch;
     float* vs = ks + R * pitch;
-    const int32_t m = blockIdx.x / H, h = blockIdx.x % H;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    float* ps = vs + R * pitch + w * (kSaMaxRP * kSaPP);
     const int64_t row0 = (int64_t)m * R;
     for (int i = threadIdx.x; i < R * hd; i += kSaWaves * 64) {
         const int r = i / hd, c = i % hd;
@@ -143,56 +167,95 @@ __global__ __launch_bounds__(kSaWaves * 64) void k_sa_attention(
     __syncthreads();
     const float b = beta[m], th = vth[m];
     const bool key = lane < R;
-    const int RP = min(kSaMaxRP, 64 / hd);
-    const int rr = lane / hd, cc = lane - rr * hd;  // p @ V: row rr of the group, channel cc
-    for (int i0 = w * RP; i0 < R; i0 += kSaWaves * RP) {
-        const int nr = min(RP, R - i0);
-        // the group's rows side by side (rows past R repeat row R - 1 and are
-        // not stored): their wave reductions are independent chains
-        float hn[kSaMaxRP], u[kSaMaxRP], cnt[kSaMaxRP];
-        {
-            float sd[kSaMaxRP];
+    const uint64_t keys = R == 64 ? ~0ull : (1ull << R) - 1;
+    const int rpv = 64 / hd;  // rows of a p @ V pass
+    const int rr = lane / hd, cc = lane - rr * hd;
+    float kr[HD ? HD : 1], vr[HD ? kSaMaxR : 1];
+    if constexpr (HD > 0) {
 #pragma unroll
-            for (int q = 0; q < kSaMaxRP; ++q) sd[q] = 0.0f;
-            if (key) {
+        for (int c = 0; c < HD; ++c) kr[c] = key ? ks[lane * pitch + c] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < kSaMaxR; ++j) vr[j] = j < R ? vs[j * pitch + cc] : 0.0f;
+    }
+    for (int i0 = w * NQ; i0 < R; i0 += kSaWaves * NQ) {
+        const int nr = min(NQ, R - i0);
+        // the group's rows side by side (rows past R repeat row R - 1 and are
+        // not stored): independent chains
+        float hn[NQ], u[NQ], cnt[NQ];
+        int32_t tot[NQ];
+        {
+            float sd[NQ];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) sd[q] = 0.0f;
+            if constexpr (HD > 0) {
+#pragma unroll
+                for (int c = 0; c < HD; c += 4)
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) {
+                        const float4 x = *reinterpret_cast<const float4*>(
+                                qs + min(i0 + q, R - 1) * pitch + c);
+                        sd[q] = __fadd_rn(sd[q], __fmul_rn(x.x, kr[c]));
+                        sd[q] = __fadd_rn(sd[q], __fmul_rn(x.y, kr[c + 1]));
+                        sd[q] = __fadd_rn(sd[q], __fmul_rn(x.z, kr[c + 2]));
+                        sd[q] = __fadd_rn(sd[q], __fmul_rn(x.w, kr[c + 3]));
+                    }
+            } else if (key) {
                 for (int c = 0; c < hd; ++c) {
                     const float kv = ks[lane * pitch + c];
 #pragma unroll
-                    for (int q = 0; q < kSaMaxRP; ++q)
+                    for (int q = 0; q < NQ; ++q)
                         sd[q] = __fadd_rn(sd[q], __fmul_rn(qs[min(i0 + q, R - 1) * pitch + c], kv));
                 }
             }
 #pragma unroll
-            for (int q = 0; q < kSaMaxRP; ++q) {
+            for (int q = 0; q < NQ; ++q) {
                 const float hj = key ? __fmul_rn(b, sd[q]) : 0.0f;
                 const float den = __fadd_rn(wmax(key ? fabsf(hj) : 0.0f), 1e-6f);
                 hn[q] = __fdiv_rn(hj, den);
                 u[q] = 0.0f;
                 cnt[q] = 0.0f;
+                tot[q] = 0;
             }
         }
         for (int it = 0; it < n_iter; ++it) {
 #pragma unroll
-            for (int q = 0; q < kSaMaxRP; ++q) {
-                const float G = wsum(key ? cnt[q] : 0.0f);  // integer counts: exact in any order
-                const float inh = __fmul_rn(g_inh, G);
+            for (int q = 0; q < NQ; ++q) {
+                const float inh = __fmul_rn(g_inh, (float)tot[q]);
                 float sp;
                 u[q] = lif_upd(u[q], __fsub_rn(hn[q], inh), leak, th, &sp);
                 cnt[q] = __fadd_rn(cnt[q], sp);
+                tot[q] += __popcll(__ballot(sp != 0.0f) & keys);
             }
         }
 #pragma unroll
-        for (int q = 0; q < kSaMaxRP; ++q) {
-            const float tot = wsum(key ? cnt[q] : 0.0f);
-            if (key && q < nr) ps[q * kSaPP + lane] = __fdiv_rn(cnt[q], __fadd_rn(tot, 1e-6f));
-        }
+        for (int q = 0; q < NQ; ++q)
+            if (q < nr) ps[q * kSaPP + lane] = key ? __fdiv_rn(cnt[q], __fadd_rn((float)tot[q], 1e-6f)) : 0.0f;
         // the group's weights are read by other lanes of this wave only
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        if (rr < nr) {
-            float s = 0.0f;
-            for (int j = 0; j < R; ++j) s = __fadd_rn(s, __fmul_rn(ps[rr * kSaPP + j], vs[j * pitch + cc]));
-            out[(row0 + i0 + rr) * ld + (int64_t)h * hd + cc] = s;
+        for (int q0 = 0; q0 < nr; q0 += rpv) {
+            const int q = q0 + rr;
+            if (rr < rpv && q < nr) {
+                float s = 0.0f;
+                const float* pr = ps + q * kSaPP;
+                if constexpr (HD > 0) {
+#pragma unroll
+                    for (int j = 0; j < kSaMaxR; j += 16) {
+                        if (j >= R) break;  // past R p and v are 0, and s is never -0
+#pragma unroll
+                        for (int e = 0; e < 16; e += 4) {
+                            const float4 x = *reinterpret_cast<const float4*>(pr + j + e);
+                            s = __fadd_rn(s, __fmul_rn(x.x, vr[j + e]));
+                            s = __fadd_rn(s, __fmul_rn(x.y, vr[j + e + 1]));
+                            s = __fadd_rn(s, __fmul_rn(x.z, vr[j + e + 2]));
+                            s = __fadd_rn(s, __fmul_rn(x.w, vr[j + e + 3]));
+                        }
+                    }
+                } else {
+                    for (int j = 0; j < R; ++j) s = __fadd_rn(s, __fmul_rn(pr[j], vs[j * pitch + cc]));
+                }
+                out[(row0 + i0 + q) * ld + (int64_t)h * hd + cc] = s;
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -271,10 +334,19 @@ extern "C" int hses_sa_encode(const float* d_cq, const float* d_ck, const float*
     HSES_REQUIRE(d_cq && d_ck && d_cv && d_th_q && d_th_k && d_th_v && d_pos && d_X, "NULL pointer");
     HSES_REQUIRE(d_X != d_cq && d_X != d_ck && d_X != d_cv, "X must not alias the currents");
     HSES_REQUIRE((M * d + 255) / 256 < (1ll << 31), "grid too large");
-    hipLaunchKernelGGL(k_sa_encode, dim3(blocks256(M * d)), dim3(256), 0, (hipStream_t)stream,
-                       d_cq, d_ck, d_cv, T, M, d, rows_per_member, d_th_q, d_th_k, d_th_v,
-                       1.0f / tau_m, d_pos,
-                       pos_per_member, d_X);
+    const uintptr_t bases = reinterpret_cast<uintptr_t>(d_cq) | reinterpret_cast<uintptr_t>(d_ck) |
+                            reinterpret_cast<uintptr_t>(d_cv) | reinterpret_cast<uintptr_t>(d_pos) |
+                            reinterpret_cast<uintptr_t>(d_X);
+    const bool vec = d % 4 == 0 && bases % 16 == 0;
+    auto launch = [&](auto kernel, int64_t threads) {
+        hipLaunchKernelGGL(kernel, dim3(blocks256(threads)), dim3(256), 0, (hipStream_t)stream, d_cq,
+                           d_ck, d_cv, T, M, d, rows_per_member, d_th_q, d_th_k, d_th_v, 1.0f / tau_m,
+                           d_pos, pos_per_member, d_X);
+    };
+    if (vec)
+        launch(k_sa_encode<4>, M * d / 4);
+    else
+        launch(k_sa_encode<1>, M * d);
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }
@@ -292,9 +364,17 @@ extern "C" int hses_sa_attention(const float* d_q, const float* d_k, const float
     HSES_REQUIRE(d_q && d_k && d_v && d_beta && d_vth && d_out, "NULL pointer");
     HSES_REQUIRE(d_out != d_q && d_out != d_k && d_out != d_v, "out must not alias q, k or v");
     HSES_REQUIRE(n * H < (1ll << 31), "grid too large");
-    hipLaunchKernelGGL(k_sa_attention, dim3((uint32_t)(n * H)), dim3(kSaWaves * 64), sa_lds_bytes(R, hd),
-                       (hipStream_t)stream, d_q, d_k, d_v, ld, R, H, hd, d_beta, d_vth, g_inh,
-                       1.0f / tau_m, n_iter, d_out);
+    auto launch = [&](auto kernel, int nq, int pitch) {
+        const size_t lds = ((size_t)kSaWaves * nq * kSaPP + 3 * (size_t)R * pitch) * sizeof(float);
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)(n * H)), dim3(kSaWaves * 64), lds, (hipStream_t)stream,
+                           d_q, d_k, d_v, ld, R, H, hd, d_beta, d_vth, g_inh, 1.0f / tau_m, n_iter, d_out);
+    };
+    switch (hd) {  // 8: eight rows fill a p @ V pass
+        case 8: launch(k_sa_attention<8, 8>, 8, hd + 4); break;
+        case 16: launch(k_sa_attention<16, 4>, 4, hd + 4); break;
+        case 32: launch(k_sa_attention<32, 4>, 4, hd + 4); break;
+        default: launch(k_sa_attention<0, 4>, 4, hd + 1); break;
+    }
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }
