@@ -810,17 +810,18 @@ static int32_t f32_bn(int32_t a) { return a <= 32 ? 32 : a <= 64 ? 64 : 128; }
 static int32_t f32_rk(int32_t r) { return r <= 1 ? 1 : r <= 4 ? 4 : r <= 8 ? 8 : 16; }
 static int32_t f32_pad(int32_t a) { return (a + f32_bn(a) - 1) / f32_bn(a) * f32_bn(a); }
 
-// k_gemm_f32s takes do_Tmm (which k_gemm_f32 does not) and do_mm with at least
-// 256 outputs, over more than two K chunks (at b <= 64 a call is bound by its x
-// and y bytes).  Narrower do_mm outputs are the spiking layers': their currents
+// k_gemm_f32s takes do_Tmm (which k_gemm_f32 does not; against k_linear_small, which
+// draws a tile's factors in every tile, 1776 rows 64 -> 256 at rank 1 39 -> 13 us, 25600
+// rows 64 -> 512 at rank 2 276 -> 54 us) and do_mm with at least 256 outputs over more
+// than two K chunks (at b <= 64 such a call is bound by its x and y bytes).  Narrower do_mm outputs are the spiking layers': their currents
 // stay on the fp32 chain, because a current at the LIF threshold would spike or
 // not with the order of its sum.  The rule is the same for every x format
 // (binary inputs give the same bits in all of them).
 static bool f32_split_shape(int32_t a, int32_t b, bool tmm) {
-    return b > 2 * KF_BK && (tmm || a >= 256);
+    return tmm || (b > 2 * KF_BK && a >= 256);
 }
 static size_t f32_w_bytes(int32_t a, int32_t b) {
-    return b > 2 * KF_BK ? (size_t)((b + KF_BK - 1) / KF_BK) * 3 * f32_pad(a) * KF_BK * 2 : 0;
+    return (size_t)((b + KF_BK - 1) / KF_BK) * 3 * f32_pad(a) * KF_BK * 2;
 }
 
 // Most members a bm-row tile (starting at a multiple of bm) can touch.

@@ -1,5 +1,5 @@
 """The fp32 forward on split operands (k_gemm_f32s: do_Tmm, and do_mm with at
-least 256 outputs, over inputs more than 64 wide) against float64.
+least 256 outputs over inputs more than 64 wide) against float64.
 
 Bound: a product of two bf16 parts is exact in the fp32 accumulator, the
 products left out are below 2^-25 of |x w|, and a running sum is rounded at most
@@ -41,6 +41,9 @@ def reference(x3, W, A, B, rpm, tmm):
     (70, 500, 1, 33, 130, 1, 0, 1, FMT_F32),     # do_Tmm, 64-column tile, 128 rows
     (9, 40, 2, 70, 256, 1, 1, 1, FMT_BF16),      # do_Tmm, two column tiles
     (6, 64, 2, 130, 200, 2, 0, 1, FMT_BITS),
+    (48, 37, 1, 256, 64, 1, 0, 1, FMT_F32),      # do_Tmm over two K chunks
+    (5, 50, 1, 300, 20, 4, 1, 1, FMT_F32),       # over part of one
+    (3, 100, 2, 17, 1, 1, 0, 1, FMT_BF16),       # over one input
 ])
 def test_split_against_float64(hses_gpu, n, rpm, T, out, inp, r, tid_lo, tmm, fmt):
     rng = np.random.default_rng(out + inp + r)
