@@ -21,8 +21,8 @@
 //     count rounded up to a wave.  Rank chunks are double-buffered in LDS (one
 //     barrier per chunk).  hses_es_update_rec runs the same kernel on the
 //     forward's factor record, so the two agree bit for bit.
-// Without a workspace for the record (hses_es_update_noalloc's fixed scratch, or
-// r >= 32 with a split's record past the bound) the contraction draws:
+// Without a workspace for the record (hses_es_update_noalloc's fixed scratch, a
+// caller's workspace that holds the partials alone, or r >= 32 with a split's record past the bound) the contraction draws:
 //   k_es_partial (r < 32): 128x128 tiles, fp32 MFMA, a k-chunk of 32 columns holds
 //     32 / r pairs, so every thread generates a run of stream rows per chunk.
 //   k_es_rows<.., false>: the generation of the next rank chunk is interleaved with
@@ -837,6 +837,13 @@ extern "C" size_t hses_es_update_workspace(int32_t a, int32_t b, int32_t rank, i
     return std::max(bytes(cnt), bytes(cnt + 1));
 }
 
+// The plan for a workspace of work_bytes: one that holds the partials but not the
+// record draws inside the contraction.
+static EsPlan es_plan_in(int32_t a, int32_t b, int32_t rank, int32_t n_pairs, bool draw, size_t work_bytes) {
+    const EsPlan pl = es_plan(a, b, rank, n_pairs, draw);
+    return work_bytes < pl.part_bytes + 16 + pl.rec_bytes ? es_plan(a, b, rank, n_pairs, false) : pl;
+}
+
 // The ES update into a caller's workspace: d_work of work_bytes, or, with
 // scratch_cap > 0, at most scratch_cap bytes of partials in it and no record (the
 // split count is lowered until the partials fit).  rec: the forward's record.
@@ -858,7 +865,8 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
     int32_t pair_lo, n_pairs;
     pair_range(tid_lo, n, &pair_lo, &n_pairs);
     const bool rows_k = use_rows_kernel(rank);
-    EsPlan pl = es_plan(a, b, rank, n_pairs, !rec && !scratch_cap);
+    EsPlan pl = scratch_cap ? es_plan(a, b, rank, n_pairs, false)
+                            : es_plan_in(a, b, rank, n_pairs, !rec, work_bytes);
     if (scratch_cap) {
         const size_t fit = (scratch_cap - 16) / ((size_t)len * sizeof(float));
         if (fit < 1)
@@ -1022,7 +1030,7 @@ extern "C" int hses_es_update(const float* d_f, int32_t n, int32_t tid_lo, uint6
     if (n != 0 && rank != 0 && sigma != 0.0f) {
         int32_t lo, cnt;
         pair_range(tid_lo, n, &lo, &cnt);
-        const EsPlan pl = es_plan(a, b, rank, cnt, true);
+        const EsPlan pl = es_plan_in(a, b, rank, cnt, true, work_bytes);
         HSES_REQUIRE(d_f, "fitness is NULL");
         HSES_REQUIRE(d_work && work_bytes >= pl.part_bytes + 16 + pl.rec_bytes, "workspace too small");
     }

@@ -12,7 +12,8 @@ import numpy as np
 import pytest
 import torch
 
-from tests.test_gpu_update import gpu_grad, oracle_grad
+from hyperscalees_amd import _lib
+from tests.test_gpu_update import KEY, gpu_grad, oracle_grad
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +54,28 @@ def test_zero_fitness_and_scale_range(hses_gpu):
     for e in (-60, 60):
         g = gpu_grad(hses_gpu, 0.1, 2, base * np.float32(2.0 ** e), 40, 50, np.float32(2.0 ** -e))
         assert np.abs(g.cpu().numpy() - ref).max() <= 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("a,b,r,n,splits", [
+    (64, 64, 8, 1024, 64),      # k_es_partial's splits: 512 pairs / 8
+    (200, 500, 48, 302, 18),    # k_es_rows': 151 pairs / 8
+])
+def test_workspace_of_partials_alone(hses_gpu, a, b, r, n, splits):
+    """A workspace that holds the partials and the scale but no record draws inside
+    the contraction; one too small for the partials is refused."""
+    fit = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    ref = oracle_grad(0.02, r, fit, a, b, 0)
+    f, g = torch.from_numpy(fit).cuda(), torch.empty((a, b), device="cuda")
+    work = torch.empty(splits * a * b * 4 + 16, dtype=torch.uint8, device="cuda")
+
+    def call(nbytes):
+        _lib.call("hses_es_update", f.data_ptr(), n, 0, KEY & (2 ** 64 - 1), r, 0.02, 0, 0, a, b, 1.0, 0,
+                  g.data_ptr(), work.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+
+    call(work.numel())
+    K = n // 2 * r
+    tol = (2.0 ** -20 + 2.0 ** -24 * math.sqrt(K)) * math.sqrt(K) * max(np.sqrt((ref ** 2).mean()),
+                                                                        np.abs(ref).max() / 8)
+    assert np.abs(g.cpu().numpy() - ref).max() <= tol
+    with pytest.raises(_lib.HsesError):
+        call(a * b * 4)
