@@ -29,6 +29,7 @@ sys.path.insert(0, ROOT)
 METRIC = "perturbed member-evals/sec + ES-update GB/s, SNN-MLP N=8192 r=128"
 PEAK_BF16_TFLOPS = 2500.0     # MI355X dense bf16 MFMA
 PEAK_FP32_TFLOPS = 157.3      # MI355X dense fp32 MFMA
+PEAK_SPLIT3_TFLOPS = round(2500.0 / 6, 1)  # fp32 products as six bf16 ones (dense bf16 peak 2500)
 PEAK_HBM_GBPS = 8000.0
 # HBM bytes per launch of fc1's GEMM on member weights (k_mw_bits), from two rocprofv3 PMC runs
 # of `python3 -m hyperscalees_amd.profile_fc1` (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, factors
@@ -192,7 +193,7 @@ def bench_c5(args):
                    "parallelism": "single GPU"},
         "phase_ms": {"forward": round(t_fwd, 3), "es_update": round(t_upd, 3)},
         "fwd_tflops": round(rwkv_lm.forward_flops(cfg) / (t_fwd * 1e-3) / 1e12, 1),
-        "roofline": {"kernel": ("k_gemm_bf16<BF16 x, rank 1, relu^2, bf16 y> with its W->bf16 "
+        "roofline": {"kernel": ("k_gemm_bf16_dl<BF16 x> (rank 1, relu^2, bf16 y) with its W->bf16 "
                                 "conversion and factor draw (ChannelMixing key, 262144 x 512 -> "
                                 "2048)"),
                      "bound": "mfma", "achieved": round(achieved, 1), "peak": PEAK_BF16_TFLOPS,
@@ -410,7 +411,7 @@ def bench_c1(args):
         "value": round(cfg.n / (ms * 1e-3), 1), "unit": "member-evals/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "fp32 (fp32 MFMA forward and ES update)", "data": "synthetic",
+        "dtype": "fp32 (fp32 MFMA forward; ES update on fp16 split operands)", "data": "synthetic",
         "config": {"workload": ("C1: SNN-MLP 784-128-128-128-10, LIF decay 0.9 v_th 1.0, Poisson "
                                 "T=8, N=256, r=4, sigma 0.02, the same 64 inputs (70% zeros) for "
                                 "every member, full ES step (forward + fitness + z-score + ES "
@@ -468,17 +469,17 @@ def bench_c2(args):
         "value": round(n / (ms * 1e-3), 1), "unit": "member-evals/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "fp32 (fp32 MFMA forward and ES update)", "data": "synthetic",
+        "dtype": "fp32 (forward on three-way bf16 split operands, ES update on fp16 split operands)", "data": "synthetic",
         "config": {"workload": ("C2: W 1024x1024 ~ N(0, 1/32^2), N=4096, r=1, 16 rows per member, "
                                 "x ~ N(0,1); perturbed forward + z-score of N(0,1) fitness + ES "
                                 "update"),
                    "population": n, "rank": r, "parallelism": "single GPU"},
         "phase_ms": {"forward": round(fwd_ms, 4), "es_update": round(upd_ms, 4)},
         "es_update_tflops": round(upd_fl / (upd_ms * 1e-3) / 1e12, 2),
-        "roofline": {"kernel": ("k_factors + k_gemm_f32<F32 x, 128 columns, rank 1> (65536 x 1024 "
-                                "-> 1024)"),
-                     "bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_FP32_TFLOPS,
-                     "unit": "TFLOP/s", "frac": round(achieved / PEAK_FP32_TFLOPS, 4),
+        "roofline": {"kernel": ("k_factors + k_gemm_f32s<F32 x, 128 x 128, rank 1> (65536 x 1024 "
+                                "-> 1024; six bf16 products per fp32 product)"),
+                     "bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_SPLIT3_TFLOPS,
+                     "unit": "TFLOP/s", "frac": round(achieved / PEAK_SPLIT3_TFLOPS, 4),
                      "traffic": None, "launch_ms": round(fwd_ms, 4),
                      "algorithmic_flop_per_launch": fwd_fl},
     }
