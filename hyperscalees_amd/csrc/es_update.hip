@@ -495,7 +495,7 @@ __global__ __launch_bounds__(R_MAXT) void k_es_rows(UpdParams P, RowTiles G) {
 // [(pair - pair0) * r + c][stream row].  A thread draws rc consecutive rows of one
 // pair after one jump.  WEIGHT (k_es_gemm): the A rows (stream rows b ..) are
 // stored as (v * bs) * w with the pair's weight w, the reference's fp32 products,
-// and the last block writes {S, 1/S} (k_es_scale) to scale.  Bound by the draw's
+// and the last block writes {S, 1/S} (k_es_scale) and k_es_gemm's fp32 flag to scale.  Bound by the draw's
 // vector instructions (106 per normal, 300 G normals/s).
 template <bool WEIGHT>
 __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int32_t pairs, int32_t groups,
@@ -513,8 +513,10 @@ __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int
         if (threadIdx.x == 0) {
             m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
             int e;
-            scale[0] = scale_exponent(2.0f * m * fabsf(P.bs) * 6.5f, &e);  // bound on |w_p * Ahat|
+            const float top = 2.0f * m * fabsf(P.bs) * 6.5f;  // bound on |w_p * Ahat|
+            scale[0] = scale_exponent(top, &e);
             scale[1] = ldexpf(1.0f, -e);
+            scale[2] = isfinite(top) ? 0.0f : 1.0f;  // no finite operand halves (S = 1): k_es_gemm on fp32 chains
         }
         return;
     }
@@ -590,11 +592,28 @@ __global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
     // K chunks [c0, c1) of this split, as k (the last chunk of all may be short)
     const int32_t c0 = split_begin(G.chunks, P.splits, s), c1 = split_begin(G.chunks, P.splits, s + 1);
     const float S = P.scale[0];
+    const int64_t rows = (int64_t)P.a + P.b;
+    if (P.scale[2] != 0.0f) {
+        // An infinite weight, or one whose terms may pass fp32's range, has no operand
+        // halves (inf - inf): plain fp32 chains give what fp32 gives.  Thread: one
+        // column, every other row of the tile.
+        const int32_t q = tid & 127;
+        const int64_t ka = (int64_t)c0 * U_CW, ke = min((int64_t)c1 * U_CW, G.k_all);
+        for (int32_t o = tid >> 7; o < at && q < bt; o += 2) {
+            float sum = 0.0f;
+#pragma unroll 1
+            for (int64_t k = ka; k < ke; ++k) {
+                const float* col = P.rec + (k - G.rec_k0) * rows;
+                sum = __builtin_fmaf(col[P.b + o0 + o], col[q0 + q], sum);
+            }
+            P.work[(size_t)s * P.a * P.b + (size_t)(o0 + o) * P.b + q0 + q] = sum;
+        }
+        return;
+    }
     const bool is_a = tid < 128;
     const int32_t lr = is_a ? tid : tid - 128;
     const bool on = lr < (is_a ? at : bt);
     const float sc = is_a ? S : 1.0f;
-    const int64_t rows = (int64_t)P.a + P.b;
     const float* src = P.rec + (on ? (is_a ? P.b + o0 + lr : q0 + lr) : 0);
     float pv[U_CW];
     auto load = [&](int32_t ch) {

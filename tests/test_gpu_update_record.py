@@ -79,3 +79,27 @@ def test_workspace_of_partials_alone(hses_gpu, a, b, r, n, splits):
     assert np.abs(g.cpu().numpy() - ref).max() <= tol
     with pytest.raises(_lib.HsesError):
         call(a * b * 4)
+
+
+@pytest.mark.parametrize("n,bad", [(64, np.inf), (301, -np.inf), (64, 1.0e38)])
+def test_fitness_past_the_operand_halves(hses_gpu, n, bad):
+    """One fitness that is infinite, or whose terms reach fp32's range, at rank 1:
+    infinities where fp32 chains have them, with their signs, and no NaN."""
+    fit = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    fit[5] = bad
+    a, b = 130, 200
+    g = gpu_grad(hses_gpu, 1.0, 1, fit, a, b, np.float32(1.0)).cpu().numpy()
+    lone = np.zeros(n, np.float32)
+    lone[5] = np.sign(bad)
+    sign = oracle_grad(1.0, 1, lone, a, b)  # member 5's term
+    assert not np.isnan(g).any() and (np.abs(sign) > 0).all()
+    if np.isinf(bad):
+        assert np.array_equal(g, np.sign(sign) * np.float32(np.inf))
+    else:
+        big = np.abs(sign) > 1e-3  # against which the other members' terms vanish
+        ref = sign * 1.0e38       # its A operands stay below fp32's largest
+        safe = big & (np.abs(ref) < 3.3e38)
+        over = np.abs(ref) > 3.5e38
+        assert safe.any() and over.any()
+        assert np.allclose(g[safe], ref[safe], rtol=2.0 ** -21)  # three roundings
+        assert np.array_equal(g[over], np.sign(sign[over]) * np.float32(np.inf))
