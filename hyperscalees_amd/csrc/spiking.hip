@@ -4,6 +4,7 @@
 // and stores of a time plane are contiguous across the wave, and the packed
 // spike format is one __ballot per (time step, row, 64 columns) written by a
 // single lane.
+#include "lif_rows.h"
 #include "runtime.h"
 #include "spike_fmt.h"
 
@@ -601,7 +602,6 @@ __global__ __launch_bounds__(256) void k_lif4(const float* __restrict__ cur,
 // 10000 rows of 130, T = 20: 38 -> 29 us (119 MB, 4.1 TB/s; a copy reaches 4.76) against
 // the one-column kernel, which keeps rows with gaps, widths past 512 and T past 64.
 typedef f32x4v f32x4u __attribute__((aligned(4)));
-constexpr int kLifRowsThreads = 512, kLifRowsMaxT = 64;
 __global__ __launch_bounds__(kLifRowsThreads) void k_lif_rows(
         const float* __restrict__ cur, const float* __restrict__ v0, int32_t T, int64_t rows, int32_t h,
         int32_t RB, float leak, float v_th, uint64_t* __restrict__ spk, int64_t spk_stride,
@@ -612,12 +612,9 @@ __global__ __launch_bounds__(kLifRowsThreads) void k_lif_rows(
     const int64_t row0 = (int64_t)blockIdx.x * RB;
     const int32_t rb = (int32_t)min<int64_t>(RB, rows - row0);
     const int64_t plane = rows * h;
-    // RB is a multiple of 4, so only the plane's last columns can be fewer than four:
-    // their thread loads the plane's last four and drops the `over` that are its
-    // neighbour's.  Threads past the run repeat its first columns.
-    const int32_t own = rb * h - 4 * tid;  // columns from this thread's first to the run's end
-    const int32_t over = own > 0 && own < 4 ? 4 - own : 0;
-    const int64_t e = row0 * h + (own > 0 ? 4 * tid - over : 0);
+    const LifCols cols = lif_rows_cols(row0, rb, h, tid, plane);
+    const int32_t own = cols.own, over = cols.over;
+    const int64_t e = cols.e;
     f32x4v v = v0 ? (f32x4v)*reinterpret_cast<const f32x4u*>(v0 + e) : f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
     auto step = [&](int c4, float c) {
         // snn.rs:61-63: charged = v + ((-v) + c) * leak; each op rounds.
@@ -666,18 +663,6 @@ __global__ __launch_bounds__(kLifRowsThreads) void k_lif_rows(
         if (left < 64u) x &= (1ull << left) - 1;
         spk[((int64_t)t * rows + row0 + r) * spk_stride + w] = x;
     }
-}
-
-// Rows of a k_lif_rows block: the first multiple of 4 whose threads fill 7/8 of their
-// waves, or the fullest; 0 where four rows are too wide.
-static int32_t lif_rows_block(int32_t h) {
-    int32_t best = 0, best_fill = 0;
-    for (int32_t rb = 4; (int64_t)rb * h / 4 <= kLifRowsThreads; rb += 4) {
-        const int32_t lanes = rb * h / 4, fill = lanes * 256 / ((lanes + 63) & ~63);
-        if (fill > best_fill) best = rb, best_fill = fill;
-        if (fill >= 224) break;
-    }
-    return best;
 }
 
 // snn.rs:274: spikes.mean_dim(0) -- the count of spikes over T divided by T.
@@ -941,7 +926,7 @@ extern "C" int hses_lif_scan(const float* d_cur, const float* d_v0, int32_t T, i
     }
     const int32_t rb = lif_rows_block(h);
     if (fmt == HSES_FMT_BITS && rb && cur_stride == h && rows * h >= 4 && T >= 1 && T <= kLifRowsMaxT) {
-        const int32_t threads = (rb * h / 4 + 63) & ~63;
+        const int32_t threads = lif_rows_threads(rb, h);
         hipLaunchKernelGGL(k_lif_rows, dim3((uint32_t)((rows + rb - 1) / rb)), dim3(threads),
                            (size_t)T * (threads / 16 + 1) * 8, s, d_cur, d_v0, T, rows, h, rb, leak, v_th,
                            static_cast<uint64_t*>(d_spikes), spk_stride, d_v_out);

@@ -21,6 +21,10 @@ pytestmark = pytest.mark.gpu
     (3, 5, 511, 3, 0),       # widest with four rows a block; a block of one row
     (5, 700, 10, 0, 0),      # six rows a word
     (2, 4, 1, 1, 0),         # four columns in all
+    (6, 225, 1, 0, 0),       # last blocks of one, two and three columns: most threads idle
+    (5, 226, 1, 1, 0),
+    (3, 77, 3, 0, 1),
+    (7, 113, 2, 2, 0),
     (65, 6, 100, 0, 0),      # past the longest: the one-column kernel
     (4, 5, 513, 0, 0),       # too wide for a run: the one-column kernel
 ])
