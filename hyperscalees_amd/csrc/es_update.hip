@@ -512,11 +512,14 @@ __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int
         __syncthreads();
         if (threadIdx.x == 0) {
             m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-            int e;
+            int e = 0;
             const float top = 2.0f * m * fabsf(P.bs) * 6.5f;  // bound on |w_p * Ahat|
-            scale[0] = scale_exponent(top, &e);
+            // Past these bounds (infinite fitness among it) no power of two that fp32
+            // holds puts the terms into fp16's range: S = 1 and k_es_gemm on fp32 chains.
+            const bool halves = m == 0.0f || (top >= 0x1p-85f && top <= 0x1p115f);
+            scale[0] = halves ? scale_exponent(top, &e) : 1.0f;
             scale[1] = ldexpf(1.0f, -e);
-            scale[2] = isfinite(top) ? 0.0f : 1.0f;  // no finite operand halves (S = 1): k_es_gemm on fp32 chains
+            scale[2] = halves ? 0.0f : 1.0f;
         }
         return;
     }
@@ -594,9 +597,9 @@ __global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
     const float S = P.scale[0];
     const int64_t rows = (int64_t)P.a + P.b;
     if (P.scale[2] != 0.0f) {
-        // An infinite weight, or one whose terms may pass fp32's range, has no operand
-        // halves (inf - inf): plain fp32 chains give what fp32 gives.  Thread: one
-        // column, every other row of the tile.
+        // Infinite weights, or terms that cannot be scaled into fp16's range, have no
+        // operand halves: plain fp32 chains give what fp32 gives.  Thread: one column,
+        // every other row of the tile.
         const int32_t q = tid & 127;
         const int64_t ka = (int64_t)c0 * U_CW, ke = min((int64_t)c1 * U_CW, G.k_all);
         for (int32_t o = tid >> 7; o < at && q < bt; o += 2) {

@@ -81,6 +81,26 @@ def test_workspace_of_partials_alone(hses_gpu, a, b, r, n, splits):
         call(a * b * 4)
 
 
+@pytest.mark.parametrize("a,b,r,n,e", [
+    (40, 50, 2, 64, -100), (40, 50, 2, 64, 100),    # 2^e alone is a scale fp32 holds
+    (40, 50, 2, 64, -115), (40, 50, 2, 64, 119),    # a scale that is not
+    (130, 70, 1, 301, -110), (130, 70, 1, 301, 118),
+    (20, 140, 16, 33, -112), (20, 140, 16, 33, 120),
+])
+def test_fitness_near_the_ends_of_fp32(hses_gpu, a, b, r, n, e):
+    """A finite fitness whose terms are near fp32's ends gives the scaled gradient."""
+    base = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    ref = oracle_grad(0.1, r, base, a, b)
+    g = gpu_grad(hses_gpu, 0.1, r, base * np.float32(2.0 ** e), a, b, np.float32(2.0 ** -e)).cpu().numpy()
+    assert np.isfinite(g).all()
+    # a fp32 chain of K terms: 2^-24 sqrt(K) of the sum of |terms|, below sqrt(K) times
+    # the gradient's root mean square; and three roundings of a term
+    K = (n + 1) // 2 * r
+    tol = 2.0 ** -24 * (math.sqrt(K) + 4) * math.sqrt(K) * max(np.sqrt((ref ** 2).mean()),
+                                                               np.abs(ref).max() / 8)
+    assert np.abs(g - ref).max() <= tol, (np.abs(g - ref).max(), tol)
+
+
 @pytest.mark.parametrize("n,bad", [(64, np.inf), (301, -np.inf), (64, 1.0e38)])
 def test_fitness_past_the_operand_halves(hses_gpu, n, bad):
     """One fitness that is infinite, or whose terms reach fp32's range, at rank 1:
