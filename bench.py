@@ -411,7 +411,7 @@ def bench_c1(args):
         "value": round(cfg.n / (ms * 1e-3), 1), "unit": "member-evals/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "fp32 (fp32 MFMA forward; ES update on fp16 split operands)", "data": "synthetic",
+        "dtype": "fp32 (fp32 MFMA forward; ES update on three-way bf16 split operands)", "data": "synthetic",
         "config": {"workload": ("C1: SNN-MLP 784-128-128-128-10, LIF decay 0.9 v_th 1.0, Poisson "
                                 "T=8, N=256, r=4, sigma 0.02, the same 64 inputs (70% zeros) for "
                                 "every member, full ES step (forward + fitness + z-score + ES "
@@ -469,7 +469,7 @@ def bench_c2(args):
         "value": round(n / (ms * 1e-3), 1), "unit": "member-evals/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "fp32 (forward on three-way bf16 split operands, ES update on fp16 split operands)", "data": "synthetic",
+        "dtype": "fp32 (forward and ES update on three-way bf16 split operands)", "data": "synthetic",
         "config": {"workload": ("C2: W 1024x1024 ~ N(0, 1/32^2), N=4096, r=1, 16 rows per member, "
                                 "x ~ N(0,1); perturbed forward + z-score of N(0,1) fitness + ES "
                                 "update"),

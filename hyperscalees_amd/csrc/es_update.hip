@@ -15,7 +15,8 @@
 // contracted from there; drawing inside the contraction repeated every row's
 // draw in each output tile that needs it (8 times at 1024 x 1024).
 //   k_es_draw   one thread per run of stream rows; coalesced over the rows.
-//   r < 32: k_es_gemm  128 x 128 output tiles, split over K chunks of 32.
+//   r < 32: k_es_gemm  128 x 128 output tiles, split over K chunks of 32, on three bf16
+//     parts per operand.
 //   r >= 32: k_es_rows<.., true>  one thread per stream row.  A tile spans up to
 //     128 rows of a and up to 384 columns of b, with blockDim = the tile's row
 //     count rounded up to a wave.  Rank chunks are double-buffered in LDS (one
@@ -56,7 +57,7 @@ struct UpdParams {
     int32_t pair_lo, n_pairs, splits;
     int32_t rc;  // stream rows per generation item (small ranks)
     float* work;
-    const float* scale;  // k_es_rows: {S, 1/S} (device)
+    const float* scale;  // k_es_rows: {S, 1/S}; k_es_gemm: its fp32 flag (device)
     const BmTables* tables;
     const uint32_t* log_exc;
     const uint32_t* cos_exc;
@@ -205,16 +206,6 @@ __device__ __forceinline__ void split_f16x4(const float (&x)[4], uint2* hi, uint
     *lo = __builtin_bit_cast(uint2, l);
 }
 
-// 2^e, the operand scale for terms of at most `top`.
-__device__ __forceinline__ float scale_exponent(float top, int* e) {
-    *e = 0;
-    if (top > 0.0f && isfinite(top)) {
-        frexpf(32768.0f / top, e);
-        *e = min(max(*e - 1, -100), 100);  // 2^e <= 2^15 / top
-    }
-    return ldexpf(1.0f, *e);
-}
-
 // Operand scale S (a power of two) of k_es_rows, and 1/S for k_es_reduce.
 // The A operand is S * (w_p * Ahat): |Ahat| <= base_sigma * 6.44 (the largest
 // Box-Muller radius, u1 >= 2^-24) and |w_p| <= 2 max|f|, so S puts the largest
@@ -232,8 +223,13 @@ __global__ __launch_bounds__(1024) void k_es_scale(const float* __restrict__ f, 
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        int e;
-        out[0] = scale_exponent(2.0f * red[0] * fabsf(bs) * 6.5f, &e);  // bound on |w_p * Ahat|
+        const float top = 2.0f * red[0] * fabsf(bs) * 6.5f;  // bound on |w_p * Ahat|
+        int e = 0;
+        if (top > 0.0f && isfinite(top)) {
+            frexpf(32768.0f / top, &e);
+            e = min(max(e - 1, -100), 100);  // 2^e <= 2^15 / top
+        }
+        out[0] = ldexpf(1.0f, e);
         out[1] = ldexpf(1.0f, -e);
     }
 }
@@ -495,7 +491,7 @@ __global__ __launch_bounds__(R_MAXT) void k_es_rows(UpdParams P, RowTiles G) {
 // [(pair - pair0) * r + c][stream row].  A thread draws rc consecutive rows of one
 // pair after one jump.  WEIGHT (k_es_gemm): the A rows (stream rows b ..) are
 // stored as (v * bs) * w with the pair's weight w, the reference's fp32 products,
-// and the last block writes {S, 1/S} (k_es_scale) and k_es_gemm's fp32 flag to scale.  Bound by the draw's
+// and the last block writes k_es_gemm's fp32 flag to scale[0].  Bound by the draw's
 // vector instructions (106 per normal, 300 G normals/s).
 template <bool WEIGHT>
 __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int32_t pairs, int32_t groups,
@@ -512,14 +508,8 @@ __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int
         __syncthreads();
         if (threadIdx.x == 0) {
             m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-            int e = 0;
             const float top = 2.0f * m * fabsf(P.bs) * 6.5f;  // bound on |w_p * Ahat|
-            // Past these bounds (infinite fitness among it) no power of two that fp32
-            // holds puts the terms into fp16's range: S = 1 and k_es_gemm on fp32 chains.
-            const bool halves = m == 0.0f || (top >= 0x1p-85f && top <= 0x1p115f);
-            scale[0] = halves ? scale_exponent(top, &e) : 1.0f;
-            scale[1] = ldexpf(1.0f, -e);
-            scale[2] = halves ? 0.0f : 1.0f;
+            scale[0] = m == 0.0f || (top >= 0x1p-70f && top <= 0x1p120f) ? 0.0f : 1.0f;
         }
         return;
     }
@@ -566,27 +556,32 @@ __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int
 }
 
 // ---- k_es_gemm ------------------------------------------------------------------
-// partial[s] = sum over the split's k of (S A[o, k]) B[q, k] from k_es_draw's record
+// partial[s] = sum over the split's k of A[o, k] B[q, k] from k_es_draw's record
 // (k = pair * r + rank column from the record's first pair).  128 x 128 tiles, four
-// waves of 64 x 64 on fp16 MFMA 32x32x16 with split operands as in k_es_rows
-// (x = xh + xl; hi hi + hi lo + lo hi).  Thread t stages stream row t of the tile
-// (A rows, then B rows): its 32 k of a chunk are 32 loads, each coalesced over the
-// rows, one chunk ahead (two chunks ahead in two register sets: 62 -> 65 us); the LDS rows (hi 64 B, lo 64 B, pitch 144 B: a 16-byte
-// read's 16 lanes fall on distinct banks) are double-buffered, one barrier per
-// chunk.  1024 x 1024 at rank 1 and 4096 members (K 2048, 8 splits of 8 chunks): 30
-// us of the call's 62 (draw 27, reduction 11; 202 us drawing in the contraction),
-// the conversions to operand halves about as long as the MFMAs.
+// waves of 64 x 64 on bf16 MFMA 32x32x16 with both operands as the three bf16 parts
+// of their fp32 values (split3) and six part products, as in k_gemm_f32s
+// (linear_f32.hip): the operands keep their 24 bits and fp32's range, and the small
+// products have sums of their own.  Thread t stages stream row t of the tile (A
+// rows, then B rows): its 32 k of a chunk are 32 loads, each coalesced over the
+// rows, one chunk ahead.  48 KB of LDS (64-byte rows per part, pieces swizzled by
+// slot_of) and two waves per SIMD let two workgroups share a CU, one's conversion and
+// barriers beside the other's MFMAs.  1024 x 1024 at rank 1 and 4096 members (K 2048,
+// 8 splits of 8 chunks): 40 us of the call's 69 (draw 27, reduction 11), against 202 us
+// drawing in the contraction.  On fp16 high and low parts and three products (22 bits)
+// it took 30, but the error was up to 2.4 times that of fp32 operands at few members
+// and 1.2 times at many; with the bf16 parts it is 0.3 to 1.0 of it (1 to 4096
+// members, ranks 1 to 24).
 struct GemmSplit {
     int64_t k_all, rec_k0;  // k of the whole call, and of the record's first column
     int32_t chunks;         // K chunks of the whole call
 };
-constexpr int E_HP = 72;  // LDS row pitch (halves)
+constexpr int E_ROWS = U_TA + U_TB;                  // staged rows: A's, then B's
+constexpr size_t kEsGemmLds = 3 * E_ROWS * U_CW * 2;
 
-typedef float f32x16e __attribute__((ext_vector_type(16)));
-
-__global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+void k_es_gemm(UpdParams P, GemmSplit G) {
     extern __shared__ __align__(16) unsigned char smem[];
-    uint16_t* lds = reinterpret_cast<uint16_t*>(smem);  // [2][256][E_HP]
+    uint16_t* lds = reinterpret_cast<uint16_t*>(smem);  // [3][E_ROWS][U_CW]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lc = lane & 31, kh = lane >> 5;
     const int32_t q0 = blockIdx.x * U_TB, o0 = blockIdx.y * U_TA;
@@ -594,12 +589,11 @@ __global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
     const int32_t s = P.split0 + blockIdx.z;
     // K chunks [c0, c1) of this split, as k (the last chunk of all may be short)
     const int32_t c0 = split_begin(G.chunks, P.splits, s), c1 = split_begin(G.chunks, P.splits, s + 1);
-    const float S = P.scale[0];
     const int64_t rows = (int64_t)P.a + P.b;
-    if (P.scale[2] != 0.0f) {
-        // Infinite weights, or terms that cannot be scaled into fp16's range, have no
-        // operand halves: plain fp32 chains give what fp32 gives.  Thread: one column,
-        // every other row of the tile.
+    if (P.scale[0] != 0.0f) {
+        // Terms past the range in which the parts are whole (infinite weights among
+        // them): plain fp32 chains give what fp32 gives.  Thread: one column, every
+        // other row of the tile.
         const int32_t q = tid & 127;
         const int64_t ka = (int64_t)c0 * U_CW, ke = min((int64_t)c1 * U_CW, G.k_all);
         for (int32_t o = tid >> 7; o < at && q < bt; o += 2) {
@@ -613,10 +607,9 @@ __global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
         }
         return;
     }
-    const bool is_a = tid < 128;
-    const int32_t lr = is_a ? tid : tid - 128;
+    const bool is_a = tid < U_TA;
+    const int32_t lr = is_a ? tid : tid - U_TA;
     const bool on = lr < (is_a ? at : bt);
-    const float sc = is_a ? S : 1.0f;
     const float* src = P.rec + (on ? (is_a ? P.b + o0 + lr : q0 + lr) : 0);
     float pv[U_CW];
     auto load = [&](int32_t ch) {
@@ -625,65 +618,63 @@ __global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
 #pragma unroll
         for (int c = 0; c < U_CW; ++c) pv[c] = (on && c < cn) ? src[(k0 + c) * rows] : 0.0f;
     };
-    auto store = [&](int buf) {
-        uint16_t* dst = lds + (buf * 256 + tid) * E_HP;
+    auto store = [&]() {
 #pragma unroll
-        for (int c = 0; c < U_CW; c += 8) {
-            uint2 h[2], l[2];
+        for (int pc = 0; pc < U_CW / 8; ++pc) {
+            uint32_t d[3][4];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                float x[4];
+            for (int u = 0; u < 4; ++u) {
+                uint32_t p[3];
+                split3(pv[8 * pc + 2 * u], pv[8 * pc + 2 * u + 1], p);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = pv[c + 4 * u + e] * sc;
-                split_f16x4(x, &h[u], &l[u]);
+                for (int w = 0; w < 3; ++w) d[w][u] = p[w];
             }
-            *reinterpret_cast<uint4*>(dst + c) = uint4{h[0].x, h[0].y, h[1].x, h[1].y};
-            *reinterpret_cast<uint4*>(dst + U_CW + c) = uint4{l[0].x, l[0].y, l[1].x, l[1].y};
+            const int sl = slot_of(tid, pc);
+#pragma unroll
+            for (int w = 0; w < 3; ++w)
+                *reinterpret_cast<uint4*>(lds + (w * E_ROWS + tid) * U_CW + 8 * sl) =
+                    uint4{d[w][0], d[w][1], d[w][2], d[w][3]};
         }
     };
     const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    f32x16e acc[2][2];
+    // acc: the products of the leading parts; low: the others', 2^-8 of them and less
+    f32x16 acc[2][2], low[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-    auto mfma = [](const uint4& a, const uint4& b, f32x16e c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b),
-                                                      c, 0, 0, 0);
-    };
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.0f;
     if (c0 < c1) load(c0);
     for (int32_t ch = c0; ch < c1; ++ch) {
-        const int buf = (ch - c0) & 1;
-        store(buf);
-        __syncthreads();  // also: every wave is past chunk ch - 1, whose buffer ch + 1 takes
+        if (ch > c0) __syncthreads();  // every wave is past its reads of chunk ch - 1
+        store();
+        __syncthreads();
         if (ch + 1 < c1) load(ch + 1);
-        const uint16_t* A = lds + buf * 256 * E_HP;
-        const uint16_t* B = A + 128 * E_HP;
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            const int off = 16 * ks + 8 * kh;
-            uint4 ah[2], al[2], bh[2], bl[2];
+            u16x8 af[2][3], bf[2][3];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                ah[i] = *reinterpret_cast<const uint4*>(A + (wm + 32 * i + lc) * E_HP + off);
-                al[i] = *reinterpret_cast<const uint4*>(A + (wm + 32 * i + lc) * E_HP + U_CW + off);
-                bh[i] = *reinterpret_cast<const uint4*>(B + (wn + 32 * i + lc) * E_HP + off);
-                bl[i] = *reinterpret_cast<const uint4*>(B + (wn + 32 * i + lc) * E_HP + U_CW + off);
+                const int ra = wm + 32 * i + lc, rb = U_TA + wn + 32 * i + lc;
+#pragma unroll
+                for (int p = 0; p < 3; ++p) {
+                    af[i][p] = lds_u16x8(lds + (p * E_ROWS + ra) * U_CW + 8 * slot_of(ra, 2 * ks + kh));
+                    bf[i][p] = lds_u16x8(lds + (p * E_ROWS + rb) * U_CW + 8 * slot_of(rb, 2 * ks + kh));
+                }
             }
+            // the products down to 2^-16 of the largest: a_p b_q, p + q <= 2
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int p = 0; p < 3; ++p)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = mfma(ah[i], bh[j], acc[i][j]);
+                for (int q = 0; q < 3 - p; ++q)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+                    for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = mfma(ah[i], bl[j], acc[i][j]);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = mfma(al[i], bh[j], acc[i][j]);
+                        for (int j = 0; j < 2; ++j) {
+                            if (p + q == 0) acc[i][j] = mfma_bf(af[i][p], bf[j][q], acc[i][j]);
+                            else low[i][j] = mfma_bf(af[i][p], bf[j][q], low[i][j]);
+                        }
         }
     }
     // element e of lane l: row 8 (e / 4) + 4 kh + e % 4 of the 32-row tile, column lc
@@ -697,7 +688,8 @@ __global__ __launch_bounds__(256) void k_es_gemm(UpdParams P, GemmSplit G) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int row = wm + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
-                if (row < at) out[(size_t)(o0 + row) * P.b + q0 + col] = acc[i][j][e];
+                if (row < at)
+                    out[(size_t)(o0 + row) * P.b + q0 + col] = __fadd_rn(acc[i][j][e], low[i][j][e]);
             }
         }
 }
@@ -1000,7 +992,7 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
             if (rows_k)
                 hipLaunchKernelGGL(k_es_draw<false>, dim3((uint32_t)blocks), dim3(256), 0, s, D, p0,
                                    p1 - p0, groups, d_rec, vec, d_scale);
-            else  // its last block writes the operand scale
+            else  // its last block writes k_es_gemm's flag
                 hipLaunchKernelGGL(k_es_draw<true>, dim3((uint32_t)blocks + 1), dim3(256), 0, s, D, p0,
                                    p1 - p0, groups, d_rec, vec, d_scale);
             HSES_CHECK_HIP(hipGetLastError());
@@ -1010,11 +1002,8 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
                 rc = launch_rows(cnt, true);
                 if (rc) return rc;
             } else {
-                constexpr size_t lds = 2 * 256 * E_HP * 2;
-                HSES_CHECK_HIP(hipFuncSetAttribute((const void*)k_es_gemm,
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
                 const dim3 grid((b + U_TB - 1) / U_TB, (a + U_TA - 1) / U_TA, cnt);
-                hipLaunchKernelGGL(k_es_gemm, grid, dim3(256), lds, s, P,
+                hipLaunchKernelGGL(k_es_gemm, grid, dim3(256), kEsGemmLds, s, P,
                                    GemmSplit{K, (int64_t)p0 * rank, pl.chunks});
                 HSES_CHECK_HIP(hipGetLastError());
             }
@@ -1027,9 +1016,8 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
         hipLaunchKernelGGL(k_es_partial, grid, dim3(U_THREADS), 0, s, P);
         HSES_CHECK_HIP(hipGetLastError());
     }
-    const bool scaled = rows_k || pl.draw;  // the partials are S times the sums
     hipLaunchKernelGGL(k_es_reduce, dim3((uint32_t)((len + 63) / 64)), dim3(256), 0, s, P.work,
-                       P.splits, len, scale, scaled ? d_scale + 1 : nullptr, accumulate, d_grad);
+                       P.splits, len, scale, rows_k ? d_scale + 1 : nullptr, accumulate, d_grad);
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }

@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "linear_common.h"
+#include "mfma.h"
 #include "noise_dev.h"
 #include "runtime.h"
 
@@ -43,7 +44,6 @@ constexpr int KF_AMAX = 8192;      // floats of A rows a workgroup keeps for its
 constexpr int KF_RMAX = 16;        // ranks handled
 constexpr int KS_BPT = 2;          // k_gemm_f32s: B_m chunk values staged per thread
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x16 mfma32x2(float a, float b, f32x16 c) {
@@ -62,20 +62,6 @@ __device__ __forceinline__ float x_at(const void* x, int64_t off, int32_t k) {
         return static_cast<const float*>(x)[off + k];
     }
 }
-
-// The three bf16 parts of v: v = p[0] + p[1] + p[2] exactly for normal v (8 + 8
-// + 8 significant bits, each part rounded to nearest), as pairs of consecutive k.
-__device__ __forceinline__ void split3(float lo, float hi, uint32_t (&p)[3]) {
-    p[0] = pack_bf16x2(lo, hi);
-    const float l1 = lo - __uint_as_float(p[0] << 16), h1 = hi - __uint_as_float(p[0] & 0xffff0000u);
-    p[1] = pack_bf16x2(l1, h1);
-    p[2] = pack_bf16x2(l1 - __uint_as_float(p[1] << 16), h1 - __uint_as_float(p[1] & 0xffff0000u));
-}
-
-// Slot of 16-byte piece s (8 k) of row `row` in its 64-byte LDS row.  The lanes of
-// a 16-byte read are served 16 at a time over 64 banks; they read one piece of
-// 16 rows, four of each row / 4 class mod 4, which the XOR spreads over the banks.
-__device__ __forceinline__ int slot_of(int row, int s) { return s ^ ((row >> 2) & 3); }
 
 // Item i of the split of W: a piece of 8 k of one output row.
 __device__ __forceinline__ void split_w(const LinParams& P, uint16_t* Wp, int32_t a_pad, int64_t i) {
@@ -187,11 +173,6 @@ __global__ __launch_bounds__(256) void k_factors(LinParams P, int32_t rc, int32_
 }
 
 // ---- k_gemm_f32s -----------------------------------------------------------------
-__device__ __forceinline__ f32x16 mfma_bf(const u16x8& a, const u16x8& b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
 // What bounds it: the matrix cores.  The x chunk goes global -> registers (one
 // chunk ahead) -> three parts in LDS, W arrives split (its conversion would
 // repeat in every row tile); 48 KB of LDS and two waves per SIMD let two

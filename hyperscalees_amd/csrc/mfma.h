@@ -37,6 +37,29 @@ __device__ __forceinline__ f32x4 mfma_bf16(const u16x8& a, const u16x8& b, f32x4
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// The three bf16 parts of v, each rounded to nearest, as pairs of consecutive k:
+// v = p[0] + p[1] + p[2] exactly (8 + 8 + 8 significant bits) while the third part
+// stays in bf16's normal range, |v| >= 2^-102; below that bits are lost from the
+// end, and past 3.39e38 the first part is infinite.
+__device__ __forceinline__ void split3(float lo, float hi, uint32_t (&p)[3]) {
+    p[0] = pack_bf16x2(lo, hi);
+    const float l1 = lo - __uint_as_float(p[0] << 16), h1 = hi - __uint_as_float(p[0] & 0xffff0000u);
+    p[1] = pack_bf16x2(l1, h1);
+    p[2] = pack_bf16x2(l1 - __uint_as_float(p[1] << 16), h1 - __uint_as_float(p[1] & 0xffff0000u));
+}
+
+// Slot of 16-byte piece s (8 k) of row `row` in its 64-byte LDS row.  The lanes of
+// a 16-byte read are served 16 at a time over 64 banks; they read one piece of
+// 16 rows, four of each row / 4 class mod 4, which the XOR spreads over the banks.
+__device__ __forceinline__ int slot_of(int row, int s) { return s ^ ((row >> 2) & 3); }
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ f32x16 mfma_bf(const u16x8& a, const u16x8& b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 __device__ __forceinline__ u16x8 lds_u16x8(const uint16_t* p) {
     return *reinterpret_cast<const u16x8*>(p);
 }

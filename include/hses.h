@@ -505,7 +505,12 @@ int hses_perturbed_linear_lif_mw(const void *d_x, int32_t x_fmt, int64_t x_strid
  * Deterministic: a fixed split-K partition and a fixed-order second-stage
  * reduction, no atomics.  accumulate != 0 adds into d_grad (the K-chunk
  * loop of accumulated_update) instead of overwriting it.  d_work must hold
- * hses_es_update_workspace(...) bytes. */
+ * hses_es_update_workspace(...) bytes; one that holds the partial sums but not the
+ * record of the normals is taken too (the normals are then drawn again in every
+ * output tile).  Operands: below rank 32 every fp32 value as three bf16 parts (its
+ * 24 bits; six part products), or plain fp32 where a term may leave 2^-70 .. 2^120;
+ * from rank 32 on as an fp16 high and low part (22 bits, three products) with the
+ * weighted factor scaled by a power of two into fp16's range. */
 size_t hses_es_update_workspace(int32_t a, int32_t b, int32_t rank, int32_t n);
 int hses_es_update(const float *d_f, int32_t n, int32_t tid_lo, uint64_t key, int32_t rank,
                    float sigma, int32_t epoch, int32_t noise_reuse, int32_t a, int32_t b,

@@ -2,7 +2,8 @@
 rank 32 or k_es_rows) against the oracle's double-accumulated sum, at the edges of
 its tiles, K chunks and pair ranges.
 
-Bound: the split operands leave out less than 2^-20 of a term and each of the K
+Bound: the split operands leave out less than 2^-20 of a term (2^-24 below rank 32,
+where they keep 24 bits) and each of the K
 fp32 sums rounds by half an ulp of a partial sum: 2^-20 + 2^-24 sqrt(K) of the sum
 of |terms|, which by the normals' independence is below sqrt(K) times the
 gradient's root mean square per element."""
@@ -79,6 +80,20 @@ def test_workspace_of_partials_alone(hses_gpu, a, b, r, n, splits):
     assert np.abs(g.cpu().numpy() - ref).max() <= tol
     with pytest.raises(_lib.HsesError):
         call(a * b * 4)
+
+
+@pytest.mark.parametrize("a,b,n,tid_lo", [(130, 386, 1, 0), (5, 7, 1, 3), (128, 256, 2, 0), (257, 64, 2, 4)])
+def test_one_pair_keeps_fp32_operands(hses_gpu, a, b, n, tid_lo):
+    """One pair at rank 1: every output is one product of fp32 operands, within the
+    roundings of the weight, of the weighted factor and of the product (half an ulp
+    each, 2^-24) and 2^-24 for the part products left out, of |term|; the operands'
+    zeros aside, small values included."""
+    fit = np.random.default_rng(a).standard_normal(n).astype(np.float32)
+    ref = oracle_grad(0.02, 1, fit, a, b, tid_lo)
+    # odd members carry the even ones' noise negated: their terms add up
+    s = np.abs(oracle_grad(0.02, 1, np.abs(fit) * np.where(np.arange(n) % 2, -1.0, 1.0), a, b, tid_lo))
+    g = gpu_grad(hses_gpu, 0.02, 1, fit, a, b, np.float32(1.0), tid_lo).cpu().numpy()
+    assert (np.abs(g - ref) <= 4 * 2.0 ** -24 * s).all(), (np.abs(g - ref) / s).max()
 
 
 @pytest.mark.parametrize("a,b,r,n,e", [
