@@ -458,13 +458,17 @@ void k_gemm_f32s(LinParams P, const float* __restrict__ F, const uint16_t* __res
                 const int32_t col = wn0 + 32 * j + lc;
                 if (col >= ct) continue;
                 const float yv = __fadd_rn(acc[i][j][e], low[i][j][e]);
-                bad |= !(fabsf(yv) < INFINITY);
+                const float ay = fabsf(yv);
+                bad |= !(ay < INFINITY) || (ay < 0x1p-60f && ay > 0.0f);
                 yrow[col] = noisy ? add_noise(yv, row, col) : yv;
             }
         }
-    // A part of an infinity, a NaN or a magnitude that rounds up to infinity is
-    // not finite and leaves its row or column of sums so: the wave then forms
-    // its outputs again with plain fp32 chains, which give what fp32 gives.
+    // A part of an infinity, a NaN or a magnitude that rounds up to infinity is not
+    // finite and leaves its row or column of sums so.  Parts below 2^-126 lose bits
+    // (operands under 2^-102, split3): b 2^-126 times the other operand, less than
+    // the fp32 sums' own rounding where |y| >= 2^-60 and the operands are below 2^42.
+    // Past either bound the wave forms its outputs again with plain fp32 chains,
+    // which give what fp32 gives (sums of exactly 0, as of rows of zeros, stand).
     if (__any(bad)) {
 #pragma unroll 1
         for (int32_t e = lane; e < WM * WN; e += 64) {

@@ -72,6 +72,37 @@ def test_split_against_float64(hses_gpu, n, rpm, T, out, inp, r, tid_lo, tmm, fm
     assert err <= tol, f"error {err:.2e} of the sum of |terms|, bound {tol:.2e}"
 
 
+@pytest.mark.parametrize("n,inp,out,tmm,fmt,xe,we", [
+    (150, 100, 300, 0, FMT_F32, -121, 0),    # x below the parts' range
+    (70, 66, 256, 0, FMT_F32, 0, -121),      # W
+    (130, 97, 270, 0, FMT_F32, -120, 30),    # x, against large weights
+    (90, 64, 40, 1, FMT_F32, -60, -60),      # the part products
+    (129, 130, 70, 1, FMT_BF16, 0, -121),
+    (200, 80, 260, 0, FMT_BITS, 0, -121),
+])
+def test_split_small_magnitudes(hses_gpu, n, inp, out, tmm, fmt, xe, we):
+    """Operands so small that their bf16 parts lose bits keep the fp32 bar; rows of
+    zeros beside them stay zero."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, inp)).astype(np.float32)
+    x = (x > 0).astype(np.float32) if fmt == FMT_BITS else x * np.float32(2.0 ** xe)
+    x[5] = 0.0
+    xt = torch.from_numpy(x).cuda()
+    if fmt == FMT_BITS:
+        xt = pack_bits(x[None])
+    elif fmt == FMT_BF16:
+        xt = xt.to(torch.bfloat16)
+        x = xt.float().cpu().numpy()
+    W = (rng.standard_normal((inp, out) if tmm else (out, inp)) * np.float32(2.0 ** we)).astype(np.float32)
+    Wd = (W.T if tmm else W).astype(np.float64)
+    f = hses_gpu.perturbed_linear_t if tmm else hses_gpu.perturbed_linear
+    y = f(xt, torch.from_numpy(W).cuda(), KEY, 0, 0.0, 0, 0, 0, n, 1, x_fmt=fmt).cpu().numpy().reshape(n, out)
+    ref, s = x.astype(np.float64) @ Wd.T, np.abs(x).astype(np.float64) @ np.abs(Wd).T
+    err = np.abs(y - ref) / np.maximum(s, 1e-300)
+    assert not y[5].any()
+    assert err.max() <= 2.0 ** -24 * (4 * np.sqrt(inp) + 8), err.max()
+
+
 def test_split_values_without_parts(hses_gpu):
     """Infinities, NaN and magnitudes that round up past bf16's range give what an
     fp32 chain gives, and leave the other rows and columns alone."""
