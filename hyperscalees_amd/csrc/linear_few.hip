@@ -66,6 +66,17 @@ __device__ __forceinline__ void few_load8(const uint16_t* p, int32_t n, bool vec
     }
 }
 
+// the 8 bits of a packed row from column k on (n of them), as 0.0 / 1.0
+__device__ __forceinline__ void few_load8(const uint64_t* row, int32_t k, int32_t n, float (&v)[8]) {
+    uint32_t byte = 0;
+    if (n > 0) {
+        byte = (uint32_t)(row[k >> 6] >> (k & 63)) & 0xffu;
+        if (n < 8) byte &= (1u << n) - 1u;  // bits past the last column may be set
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (float)((byte >> i) & 1u);
+}
+
 __device__ __forceinline__ u16x8 few_bf16(const float (&v)[8]) {
     return __builtin_bit_cast(u16x8, uint4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
                                            pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])});
@@ -150,8 +161,10 @@ __global__ __launch_bounds__(FW_THREADS) void k_linear_few(LinParams P, FewArgs 
             for (int32_t c = 0; c < r; ++c) {
                 float z = 0.0f;
                 for (int32_t k = lane; k < b; k += 64) {
-                    float x = XFMT == HSES_FMT_F32 ? static_cast<const float*>(P.x)[xo[row] + k]
-                                                   : bf2f(static_cast<const uint16_t*>(P.x)[xo[row] + k]);
+                    float x;
+                    if constexpr (XFMT == HSES_FMT_F32) x = static_cast<const float*>(P.x)[xo[row] + k];
+                    else if constexpr (XFMT == HSES_FMT_BF16) x = bf2f(static_cast<const uint16_t*>(P.x)[xo[row] + k]);
+                    else x = (float)((static_cast<const uint64_t*>(P.x)[xo[row] + (k >> 6)] >> (k & 63)) & 1u);
                     float f = bs[(size_t)k * r + c];
                     if constexpr (MATH == HSES_MATH_BF16) {
                         x = bf2f(f2bf(x));
@@ -182,8 +195,10 @@ __global__ __launch_bounds__(FW_THREADS) void k_linear_few(LinParams P, FewArgs 
             float x[8];
             if constexpr (XFMT == HSES_FMT_F32)
                 few_load8(static_cast<const float*>(P.x) + xoff[g] + k, 1, n, A.xvec, x);
-            else
+            else if constexpr (XFMT == HSES_FMT_BF16)
                 few_load8(static_cast<const uint16_t*>(P.x) + xoff[g] + k, n, A.xvec, x);
+            else
+                few_load8(static_cast<const uint64_t*>(P.x) + xoff[g], k, n, x);
             if constexpr (MATH == HSES_MATH_BF16) {
                 acc[g] = mfma_bf16(wb, few_bf16(x), acc[g]);
             } else {
@@ -228,9 +243,10 @@ __global__ __launch_bounds__(FW_THREADS) void k_linear_few(LinParams P, FewArgs 
 // Few enough rows that one tile holds them, few enough members and normals that
 // every workgroup can draw them, within the shapes the tiled small-rank kernels
 // take (members x rank <= 64 per tile).  fp32 math: the layers k_gemm_f32s takes
-// (narrower ones stay on their fp32 chains, see f32_split_shape).
+// (narrower ones stay on their fp32 chains, see f32_split_shape).  The rule is the
+// same for every x format: binary inputs give the same bits in all of them.
 int launch_linear_few(LinParams& P, DeviceState* st, hipStream_t s, int32_t act, int32_t y_fmt) {
-    if (P.total > FW_ROWS || P.x_fmt == HSES_FMT_BITS) return HSES_ERR_UNSUPPORTED;
+    if (P.total > FW_ROWS) return HSES_ERR_UNSUPPORTED;
     const bool bf = P.math == HSES_MATH_BF16;
     if (!bf && (P.b <= 64 || !(P.tmm || P.a >= 256) || y_fmt != HSES_FMT_F32)) return HSES_ERR_UNSUPPORTED;
     LinParams Q = P;
@@ -272,8 +288,9 @@ int launch_linear_few(LinParams& P, DeviceState* st, hipStream_t s, int32_t act,
     };
     using std::integral_constant;
     auto by_x = [&](auto mc) -> int {
-        return P.x_fmt == HSES_FMT_F32 ? by_g(mc, integral_constant<int, HSES_FMT_F32>{})
-                                       : by_g(mc, integral_constant<int, HSES_FMT_BF16>{});
+        return P.x_fmt == HSES_FMT_F32    ? by_g(mc, integral_constant<int, HSES_FMT_F32>{})
+               : P.x_fmt == HSES_FMT_BF16 ? by_g(mc, integral_constant<int, HSES_FMT_BF16>{})
+                                          : by_g(mc, integral_constant<int, HSES_FMT_BITS>{});
     };
     return bf ? by_x(integral_constant<int, HSES_MATH_BF16>{}) : by_x(integral_constant<int, HSES_MATH_F32>{});
 }

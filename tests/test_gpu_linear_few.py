@@ -9,8 +9,8 @@ import numpy as np
 import pytest
 import torch
 
-from hyperscalees_amd._lib import FMT_BF16, FMT_F32, MATH_BF16, MATH_F32
-from tests.test_gpu_linear import KEY, bf16_round, factors
+from hyperscalees_amd._lib import FMT_BF16, FMT_BITS, FMT_F32, MATH_BF16, MATH_F32
+from tests.test_gpu_linear import KEY, bf16_round, factors, pack_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -50,6 +50,31 @@ def test_few_rows(hses_gpu, n, rpm, T, out, inp, r, tid_lo, tmm, fmt, math):
             n_time=T, math=math).cpu().numpy().reshape(y.shape)
     tol = 2.0 ** -24 * (2 * np.sqrt(inp) + 16) * s
     assert (np.abs(got - y) <= tol).all(), (np.abs(got - y) / tol).max()
+
+
+@pytest.mark.parametrize("math", [MATH_F32, MATH_BF16])
+@pytest.mark.parametrize("n,rpm,T,out,inp,r,tid_lo,tmm", [
+    (2, 16, 1, 256, 784, 4, 0, 0),     # a layer of a few spike rows
+    (3, 5, 4, 300, 72, 1, 1, 0),       # ragged outputs, a word's first byte, time-major planes
+    (8, 8, 1, 40, 200, 2, 0, 1),       # do_Tmm
+    (4, 16, 1, 100, 136, 2, 3, 0),     # narrower outputs
+])
+def test_few_rows_formats_agree(hses_gpu, n, rpm, T, out, inp, r, tid_lo, tmm, math):
+    """Binary inputs give the same bits in every format, whatever lies past a
+    packed row's last column."""
+    rng = np.random.default_rng(out)
+    x3 = (rng.random((T, n * rpm, inp)) < 0.3).astype(np.float32)
+    xt = torch.from_numpy(x3).cuda()
+    past = np.ones((T, n * rpm, (inp + 63) // 64 * 64), np.float32)
+    past[..., :inp] = x3
+    shape = (inp, out) if tmm else (out, inp)
+    W = torch.from_numpy((rng.standard_normal(shape) / np.sqrt(inp)).astype(np.float32)).cuda()
+    f = hses_gpu.perturbed_linear_t if tmm else hses_gpu.perturbed_linear
+    ys = [f(x, W, KEY, r, 0.2, 0, 0, tid_lo, n, rpm, x_fmt=fmt, n_time=T, math=math).cpu().numpy()
+          for fmt, x in ((FMT_F32, xt), (FMT_BF16, xt.to(torch.bfloat16)), (FMT_BITS, pack_bits(x3)),
+                         (FMT_BITS, pack_bits(past)))]
+    for y in ys[1:]:
+        np.testing.assert_array_equal(ys[0], y)
 
 
 @pytest.mark.parametrize("act,f", [(1, np.tanh), (2, lambda v: 1 / (1 + np.exp(-v))),
