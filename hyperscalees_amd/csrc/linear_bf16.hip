@@ -416,6 +416,13 @@ void k_gemm_bf16(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, const
     else by_act(std::false_type{});
 }
 
+// Whether the three bf16 parts of a rank-1 operand hold all of it (zero, or a size
+// whose last part and part products stay in the normal ranges; not NaN).
+__device__ __forceinline__ bool parts_whole(float v) {
+    const float a = fabsf(v);
+    return a == 0.0f || (a >= 0x1p-50f && a <= 0x1p60f);
+}
+
 // The same product at rank 0 or 1 (see DL_BM).  x B_m and the rank-1 term are
 // matrix products, so the matrix cores form them (on the vector ALU they were
 // 2900 instructions per wave and tile, more issue time than the MFMAs):
@@ -425,7 +432,8 @@ void k_gemm_bf16(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, const
 //   (x B_m) A_m^T   one k slice at the end.  Each fp32 factor is the sum of three
 //           bf16 parts (8 significant bits each), and the six products p + q <= 2
 //           fill 6 of the 8 k of a lane: half a slice per member, so the term keeps
-//           fp32 accuracy and one rounding.
+//           fp32 accuracy and one rounding.  A tile with a factor or an x B_m
+//           outside 2^-50 .. 2^60 (parts_whole) takes fp32 products instead.
 // F: the output-side factor rows (fp32, member pitch a + b); Fb: the input-side
 // rows as bf16 (member pitch b).
 // At 100000 x 512 -> 2048 (bf16 x and y, relu^2, 100 rows per member) the call
@@ -606,10 +614,19 @@ void k_gemm_bf16_dl(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, co
 
     // ---- (x B_m) A_m^T as one k slice per two members --------------------------------
     if constexpr (NOISY) {
-        __syncthreads();  // every wave is past its last read of the stages
+        // lane lc (hl 0) of wave (wr, wc): row 64 wr + 32 wc + lc, element m its
+        // product with member m's factor
+        const int32_t xbr = 64 * wr + 32 * wc + lc;
+        const int32_t xbm = nm == 1 || xbr >= rows_here ? 0 : tr.member(P, xbr);
+        const float xb = xbm == 0 ? xba[0] : xbm == 1 ? xba[1] : xbm == 2 ? xba[2] : xba[3];
+        bool plain = hl == 0 && xbr < rows_here && !parts_whole(xb);
+#pragma unroll
+        for (int m = 0; m < DL_NM; ++m) plain |= m < nm && !parts_whole(ao[m]);
+        // every wave is past its last read of the stages
+        plain = __syncthreads_or(plain);
         uint4* AF = reinterpret_cast<uint4*>(smem);  // [nm][256] output-side fragments
         uint4* XF = AF + DL_NM * KB_BN;              // [128] x B_m fragments
-        // products k: a0 x0, a1 x0, a0 x1, a1 x1, a2 x0, a0 x2
+        // products k: a0 x0, a1 x0, a0 x1, a1 x1, a2 x0, a0 x2 (plain: the fp32 factors)
 #pragma unroll
         for (int m = 0; m < DL_NM; ++m) {
             if (m >= nm) break;
@@ -618,34 +635,31 @@ void k_gemm_bf16_dl(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, co
             const uint32_t p1 = pack_bf16x2(r1, 0.0f);
             const uint32_t p2 = pack_bf16x2(r1 - __uint_as_float(p1 << 16), 0.0f);
             const uint32_t p01 = p0 | (p1 << 16);
-            AF[m * KB_BN + tid] = uint4{p01, p01, p2 | (p0 << 16), 0u};
+            AF[m * KB_BN + tid] = plain ? uint4{__float_as_uint(ao[m]), 0u, 0u, 0u}
+                                        : uint4{p01, p01, p2 | (p0 << 16), 0u};
         }
-        // lane lc (hl 0) of wave (wr, wc): row 64 wr + 32 wc + lc, element m its
-        // product with member m's factor
-        const int32_t xbr = 64 * wr + 32 * wc + lc;
         if (hl == 0) {
-            const int32_t m = nm == 1 || xbr >= rows_here ? 0 : tr.member(P, xbr);
-            const float v = m == 0 ? xba[0] : m == 1 ? xba[1] : m == 2 ? xba[2] : xba[3];
-            // without parts (infinite, NaN, past bf16's range): its sign and size
-            // alone, so that it multiplies a0 only
-            const bool fin = fabsf(v) < 3.38e38f;
-            const uint32_t p0 = pack_bf16x2(v, 0.0f);
-            const float r1 = v - __uint_as_float(p0 << 16);
+            const uint32_t p0 = pack_bf16x2(xb, 0.0f);
+            const float r1 = xb - __uint_as_float(p0 << 16);
             const uint32_t p1 = pack_bf16x2(r1, 0.0f);
             const uint32_t p2 = pack_bf16x2(r1 - __uint_as_float(p1 << 16), 0.0f);
-            XF[xbr] = fin ? uint4{p0 | (p0 << 16), p1 | (p1 << 16), p0 | (p2 << 16), 0u}
-                          : uint4{p0, 0u, 0u, 0u};
+            XF[xbr] = plain ? uint4{__float_as_uint(xb), 0u, 0u, 0u}
+                            : uint4{p0 | (p0 << 16), p1 | (p1 << 16), p0 | (p2 << 16), 0u};
         }
         __syncthreads();
-        for (int32_t t = 0; 2 * t < nm; ++t) {
+        int32_t rm[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int32_t row = 64 * wr + 32 * i + lc;
+            rm[i] = nm == 1 || row >= rows_here ? 0 : tr.member(P, row);
+        }
+        for (int32_t t = 0; 2 * t < nm && !plain; ++t) {
             const int32_t m = 2 * t + hl;  // this lane half's member
             u16x8 xf[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const int32_t row = 64 * wr + 32 * i + lc;
-                uint4 v = XF[row];
-                const int32_t rm = nm == 1 || row >= rows_here ? 0 : tr.member(P, row);
-                if (rm != m) v = uint4{0u, 0u, 0u, 0u};
+                uint4 v = XF[64 * wr + 32 * i + lc];
+                if (rm[i] != m) v = uint4{0u, 0u, 0u, 0u};
                 xf[i] = __builtin_bit_cast(u16x8, v);
             }
 #pragma unroll
@@ -654,6 +668,21 @@ void k_gemm_bf16_dl(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, co
                 const u16x8 af = __builtin_bit_cast(u16x8, v);
 #pragma unroll
                 for (int i = 0; i < 2; ++i) acc[i][j] = mfma32b(af, xf[i], acc[i][j]);
+            }
+        }
+        if (plain) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const uint4* ar = AF + rm[i] * KB_BN + 128 * wc + 4 * hl;
+                const float x = __uint_as_float(XF[64 * wr + 32 * i + lc].x);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const float a1 = __uint_as_float(ar[32 * j + 8 * (e >> 2) + (e & 3)].x);
+                        acc[i][j][e] = __fadd_rn(acc[i][j][e], __fmul_rn(x, a1));
+                        if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // few values live at a time
+                    }
             }
         }
     }

@@ -78,3 +78,37 @@ def test_rank1_term_of_infinite_rows(hses_gpu):
             np.testing.assert_array_equal(got[row][~np.isnan(want)], want[~np.isnan(want)])
     rest = np.delete(got, [5, 70], 0)
     assert (rest == 0).all()
+
+
+@pytest.mark.parametrize("n,rpm,tmm", [(1, 128, 0), (5, 43, 0), (5, 43, 1)])
+@pytest.mark.parametrize("e", [-118, -60, 40, 127])
+def test_rank1_term_past_the_parts_range(hses_gpu, n, rpm, tmm, e):
+    """Factors whose third bf16 part is lost (sigma 2^-118) or that reach fp32's largest
+    (2^127: some are infinite) give the fp32 product of the two factors, in their own
+    member's rows alone.  W is 0, so y is the rank-1 term; x is 0 but for one value a
+    row, so x B_m is one product, exact in fp32 or rounded by the scaled side."""
+    rng = np.random.default_rng(1000 + n + e)
+    out, inp, sigma = 512, 64, 2.0 ** e
+    x = np.zeros((n * rpm, inp), np.float32)
+    cols = rng.integers(0, inp, n * rpm)
+    small = 2.0 ** -20 if e > 0 else 1.0
+    x[np.arange(n * rpm), cols] = bf16_round(rng.uniform(0.5, 2.0, n * rpm).astype(np.float32)) * np.float32(small)
+    W = torch.zeros((inp, out) if tmm else (out, inp), device="cuda")
+    f = hses_gpu.perturbed_linear_t if tmm else hses_gpu.perturbed_linear
+    got = f(torch.from_numpy(x).cuda().to(torch.bfloat16), W, KEY, 1, sigma, 0, 0, 1, n, rpm, x_fmt=FMT_BF16,
+            math=MATH_BF16).cpu().numpy().reshape(n * rpm, out)
+    with np.errstate(all="ignore"):
+        A, B = factors(sigma, 1, n, 1, inp, out) if tmm else factors(sigma, 1, n, 1, out, inp)
+        for m in range(n):
+            rows = slice(m * rpm, (m + 1) * rpm)
+            i, o = (bf16_round(A[m]), B[m]) if tmm else (bf16_round(B[m]), A[m])
+            xb = (x[rows, :].astype(np.float64) * i[:, 0].astype(np.float64)).sum(1)  # 0 x inf: NaN
+            want = xb[:, None] * o[:, 0].astype(np.float64)
+            want[np.abs(want) > 3.4028235e38 * (1 + 2.0 ** -24)] *= np.inf
+            fin = np.isfinite(want)
+            np.testing.assert_array_equal(got[rows][~fin], want[~fin].astype(np.float32))
+            # one rounding of the product (of the parts' sums: six) or an ulp of fp32's
+            # subnormals; do_Tmm sums small x A_m on the matrix cores, which may take
+            # subnormals as 0
+            least = 2.0 ** (-126 if tmm else -148)
+            assert (np.abs(got[rows] - want)[fin] <= 2.0 ** -21 * np.abs(want[fin]) + least).all()
