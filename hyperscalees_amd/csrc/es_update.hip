@@ -556,8 +556,9 @@ __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int
 }
 
 // ---- k_es_gemm ------------------------------------------------------------------
-// partial[s] = sum over the split's k of A[o, k] B[q, k] from k_es_draw's record
-// (k = pair * r + rank column from the record's first pair).  128 x 128 tiles, four
+// partial[z] = sum over the split's k of A[o, k] B[q, k] from k_es_draw's record
+// (k = pair * r + rank column from the record's first pair); a record in parts runs
+// its splits a part at a time, and each part adds to the partials of the one before.  128 x 128 tiles, four
 // waves of 64 x 64 on bf16 MFMA 32x32x16 with both operands as the three bf16 parts
 // of their fp32 values (split3) and six part products, as in k_gemm_f32s
 // (linear_f32.hip): the operands keep their 24 bits and fp32's range, and the small
@@ -574,6 +575,7 @@ __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int
 struct GemmSplit {
     int64_t k_all, rec_k0;  // k of the whole call, and of the record's first column
     int32_t chunks;         // K chunks of the whole call
+    int32_t add;            // add to the partials (of the record's parts before this one)
 };
 constexpr int E_ROWS = U_TA + U_TB;                  // staged rows: A's, then B's
 constexpr size_t kEsGemmLds = 3 * E_ROWS * U_CW * 2;
@@ -590,6 +592,7 @@ void k_es_gemm(UpdParams P, GemmSplit G) {
     // K chunks [c0, c1) of this split, as k (the last chunk of all may be short)
     const int32_t c0 = split_begin(G.chunks, P.splits, s), c1 = split_begin(G.chunks, P.splits, s + 1);
     const int64_t rows = (int64_t)P.a + P.b;
+    float* out = P.work + (size_t)blockIdx.z * P.a * P.b;
     if (P.scale[0] != 0.0f) {
         // Terms past the range in which the parts are whole (infinite weights among
         // them): plain fp32 chains give what fp32 gives.  Thread: one column, every
@@ -603,7 +606,8 @@ void k_es_gemm(UpdParams P, GemmSplit G) {
                 const float* col = P.rec + (k - G.rec_k0) * rows;
                 sum = __builtin_fmaf(col[P.b + o0 + o], col[q0 + q], sum);
             }
-            P.work[(size_t)s * P.a * P.b + (size_t)(o0 + o) * P.b + q0 + q] = sum;
+            float* w = out + (size_t)(o0 + o) * P.b + q0 + q;
+            *w = G.add ? __fadd_rn(*w, sum) : sum;
         }
         return;
     }
@@ -678,7 +682,6 @@ void k_es_gemm(UpdParams P, GemmSplit G) {
         }
     }
     // element e of lane l: row 8 (e / 4) + 4 kh + e % 4 of the 32-row tile, column lc
-    float* out = P.work + (size_t)s * P.a * P.b;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -688,8 +691,10 @@ void k_es_gemm(UpdParams P, GemmSplit G) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int row = wm + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
-                if (row < at)
-                    out[(size_t)(o0 + row) * P.b + q0 + col] = __fadd_rn(acc[i][j][e], low[i][j][e]);
+                if (row >= at) continue;
+                float* w = out + (size_t)(o0 + row) * P.b + q0 + col;
+                const float v = __fadd_rn(acc[i][j][e], low[i][j][e]);
+                *w = G.add ? __fadd_rn(*w, v) : v;
             }
         }
 }
@@ -793,6 +798,7 @@ static void pair_range(int32_t tid_lo, int32_t n, int32_t* lo, int32_t* cnt) {
 struct EsPlan {
     bool draw;
     int32_t splits, chunks, per;
+    int32_t parts;  // partial sums of an output
     size_t part_bytes, rec_bytes;
 };
 
@@ -817,7 +823,9 @@ static EsPlan es_plan(int32_t a, int32_t b, int32_t rank, int32_t n_pairs, bool 
         pl.splits = es_splits(a, b, n_pairs, rank);
     } else {
         // k_es_gemm: two workgroups per CU, at least two K chunks each, and no
-        // more k per split than the record's bound
+        // more k per split than the record's bound.  The splits of one part of the
+        // record at a time have partials: one each for all would be 16 GB at 8192 x
+        // 8192, rank 16 and 65536 members (64 parts), where one takes 256 MB.
         pl.draw = true;
         const int64_t tiles = (int64_t)((a + U_TA - 1) / U_TA) * ((b + U_TB - 1) / U_TB);
         const int64_t chunks = (K + U_CW - 1) / U_CW;
@@ -830,7 +838,8 @@ static EsPlan es_plan(int32_t a, int32_t b, int32_t rank, int32_t n_pairs, bool 
         pl.per = (int32_t)std::min<int64_t>(pl.splits, std::max<int64_t>(1, room / each));
         pairs = pl.per * each / rank + 2;
     }
-    pl.part_bytes = align_up16((size_t)pl.splits * a * b * sizeof(float));
+    pl.parts = pl.draw && !rows_k ? pl.per : pl.splits;
+    pl.part_bytes = align_up16((size_t)pl.parts * a * b * sizeof(float));
     pl.rec_bytes = pl.draw ? (size_t)(std::min<int64_t>(pairs, n_pairs) * rank * row_bytes) : 0;
     return pl;
 }
@@ -886,7 +895,7 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
         if (fit < 1)
             return set_error(HSES_ERR_INVALID_ARG, "a * b exceeds the fixed scratch of the "
                                                    "allocation-free ES update");
-        pl.splits = (int32_t)std::min<size_t>((size_t)pl.splits, fit);
+        pl.parts = pl.splits = (int32_t)std::min<size_t>((size_t)pl.splits, fit);
         pl.part_bytes = align_up16((size_t)pl.splits * len * sizeof(float));
     }
     HSES_REQUIRE(d_f, "fitness is NULL");
@@ -1004,7 +1013,7 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
             } else {
                 const dim3 grid((b + U_TB - 1) / U_TB, (a + U_TA - 1) / U_TA, cnt);
                 hipLaunchKernelGGL(k_es_gemm, grid, dim3(256), kEsGemmLds, s, P,
-                                   GemmSplit{K, (int64_t)p0 * rank, pl.chunks});
+                                   GemmSplit{K, (int64_t)p0 * rank, pl.chunks, s0 > 0});
                 HSES_CHECK_HIP(hipGetLastError());
             }
         }
@@ -1017,7 +1026,7 @@ static int es_update_impl(const float* d_f, int32_t n, int32_t tid_lo, uint64_t 
         HSES_CHECK_HIP(hipGetLastError());
     }
     hipLaunchKernelGGL(k_es_reduce, dim3((uint32_t)((len + 63) / 64)), dim3(256), 0, s, P.work,
-                       P.splits, len, scale, rows_k ? d_scale + 1 : nullptr, accumulate, d_grad);
+                       pl.parts, len, scale, rows_k ? d_scale + 1 : nullptr, accumulate, d_grad);
     HSES_CHECK_HIP(hipGetLastError());
     return HSES_OK;
 }

@@ -138,3 +138,22 @@ def test_fitness_past_the_operand_halves(hses_gpu, n, bad):
         assert safe.any() and over.any()
         assert np.allclose(g[safe], ref[safe], rtol=2.0 ** -21)  # three roundings
         assert np.array_equal(g[over], np.sign(sign[over]) * np.float32(np.inf))
+
+
+@pytest.mark.parametrize("a,b,r,n", [
+    (24, 200, 4, 320_000),    # 256 splits: the last 19 add to the first 19 partials
+    (2048, 4096, 1, 90_001),  # one split a part, three parts; the last pair is one member
+])
+def test_record_in_parts(hses_gpu, a, b, r, n):
+    """A record past its bound (512 MB) runs in parts that add to the same partials.
+    Against the sum of calls whose record is whole, with the bound above for each."""
+    fit = torch.from_numpy(np.random.default_rng(a + r).standard_normal(n).astype(np.float32)).cuda()
+    g = hses_gpu.es_update(fit, 0, KEY, r, 0.02, 0, 0, a, b, 1.0)
+    ref = torch.zeros((a, b), dtype=torch.float64, device="cuda")
+    step = (n // 4 + 1) // 2 * 2  # whole pairs
+    for lo in range(0, n, step):
+        ref += hses_gpu.es_update(fit[lo:lo + step].contiguous(), lo, KEY, r, 0.02, 0, 0, a, b, 1.0).double()
+    assert n * r * (a + b) * 2 > 512 << 20 > step * r * (a + b) * 2
+    K = n * r // 2
+    tol = 2 * (2.0 ** -20 + 2.0 ** -24 * math.sqrt(K)) * math.sqrt(K) * float((ref ** 2).mean().sqrt())
+    assert float((g.double() - ref).abs().max()) <= tol
