@@ -860,6 +860,15 @@ extern "C" size_t hses_es_update_workspace(int32_t a, int32_t b, int32_t rank, i
     return std::max(bytes(cnt), bytes(cnt + 1));
 }
 
+// The partials and {S, 1/S} alone: hses_es_update_rec is given its record.
+extern "C" size_t hses_es_update_rec_workspace(int32_t a, int32_t b, int32_t rank, int32_t n) {
+    if (a <= 0 || b <= 0 || n <= 0 || rank < U_CW) return 0;
+    int32_t lo, cnt;
+    pair_range(0, n, &lo, &cnt);
+    return std::max(es_plan(a, b, rank, cnt, false).part_bytes,
+                    es_plan(a, b, rank, cnt + 1, false).part_bytes) + 16;
+}
+
 // The plan for a workspace of work_bytes: one that holds the partials but not the
 // record draws inside the contraction.
 static EsPlan es_plan_in(int32_t a, int32_t b, int32_t rank, int32_t n_pairs, bool draw, size_t work_bytes) {

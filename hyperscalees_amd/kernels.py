@@ -587,7 +587,7 @@ def es_update_rec(fit, tid_lo, rec, rank, sigma, a, b, scale, out=None, accumula
     (the same result as es_update, without drawing the normals again)."""
     _dev(fit, torch.float32, "fit")
     n = fit.numel()
-    wbytes = _size("hses_es_update_workspace", a, b, rank, n)
+    wbytes = _size("hses_es_update_rec_workspace", a, b, rank, n)
     if work is None or work.numel() < wbytes:
         work = _workspace(wbytes, fit.device)
     if out is None:

@@ -531,7 +531,9 @@ int hses_es_update_noalloc(const float *d_f, int32_t n, int32_t tid_lo, uint64_t
 /* hses_es_update (same reference functions) of members [tid_lo, tid_lo + n)
  * reading their normals from the factor record a *_rec forward over the same
  * tid_lo and n wrote (rank >= 32): the same result, bit for bit, without
- * drawing the normals again.  Workspace: hses_es_update_workspace. */
+ * drawing the normals again.  d_work must hold hses_es_update_rec_workspace(...)
+ * bytes (the partial sums; 0 below rank 32, which the call refuses). */
+size_t hses_es_update_rec_workspace(int32_t a, int32_t b, int32_t rank, int32_t n);
 int hses_es_update_rec(const float *d_f, int32_t n, int32_t tid_lo, const float *d_rec,
                        size_t rec_bytes, int32_t rank, float sigma, int32_t a, int32_t b,
                        float scale, int32_t accumulate, float *d_grad, void *d_work,
