@@ -23,8 +23,12 @@ def _p(t):
     return t.data_ptr() if t is not None else None
 
 
+def _device():
+    return torch._C._cuda_getDevice()
+
+
 def _stream():
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return torch._C._cuda_getCurrentRawStream(_device())
 
 
 def _set_stream(s):
@@ -62,9 +66,10 @@ _SIZES = {}
 
 
 def _size(name, *shape):
-    """A size query of the library (a function of the shape alone), asked once per
-    shape; 0 is asked again (a query before hses_init may answer 0)."""
-    key = (name, shape)
+    """A size query of the library, a function of the shape and of the current device (the
+    paired factors' workspace has a slot for each of its workgroups), asked once for
+    both; 0 is asked again (a query before hses_init may answer 0)."""
+    key = (_device(), name, shape)
     n = _SIZES.get(key)
     if not n:
         if len(_SIZES) > 4096:

@@ -20,6 +20,7 @@ def test_workspace_of_an_update_from_a_record(monkeypatch):
     asked = []
     monkeypatch.setattr(K, "_dev", lambda t, dtype, name: t)
     monkeypatch.setattr(K, "_stream", lambda: 0)
+    monkeypatch.setattr(K, "_device", lambda: 0)
     monkeypatch.setattr(K, "_workspace", lambda nbytes, device: asked.append(nbytes) or torch.empty(0))
     monkeypatch.setattr(_lib, "call", lambda *args: 0)
     K.es_update_rec(torch.zeros(8192), 0, torch.zeros(1), 128, 0.02, 128, 784, 1.0)
