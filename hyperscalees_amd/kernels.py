@@ -32,9 +32,29 @@ def _stream():
 
 
 def _set_stream(s):
-    """Make torch.cuda.Stream s the current stream (the caller restores it)."""
+    """Make torch.cuda.Stream s the current stream and its device the current device."""
     torch._C._cuda_setStream(stream_id=s.stream_id, device_index=s.device_index,
                              device_type=s.device_type)
+
+
+class on_streams:
+    """with on_streams(sides, main) as turn: turn(i) makes stream i of `sides` (streams of one
+    device, taken round-robin) the current one.  At the end `main`, the caller's current
+    stream, and its device are current again, and the sides' device has the current
+    stream that it had, also where it is another device than main's."""
+
+    def __init__(self, sides, main):
+        self.sides, self.main = sides, main
+
+    def __enter__(self):
+        dev = self.sides[0].device
+        self.theirs = torch.cuda.current_stream(dev) if dev != self.main.device else None
+        return lambda i: _set_stream(self.sides[i % len(self.sides)])
+
+    def __exit__(self, *exc):
+        if self.theirs is not None:
+            _set_stream(self.theirs)
+        _set_stream(self.main)
 
 
 def _dev(t, dtype, name):

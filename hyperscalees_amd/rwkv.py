@@ -30,9 +30,10 @@ def _side_streams(dev):
 def _fan_out(jobs, inputs):
     """Run independent launches round-robin on side streams, joined into the
     current stream (a few rows: in turn on the current stream, where the joins
-    would cost more than running side by side saves).  `inputs` (made on the current stream) is recorded on the
-    side streams and every job's output on the current stream, so the caching
-    allocator reuses neither block before the stream that reads it is done."""
+    would cost more than running side by side saves).  `inputs` (made on the current
+    stream) is recorded on the side streams and every job's output on the current
+    stream, so the caching allocator reuses neither block before the stream that reads
+    it is done."""
     if inputs.shape[1] * inputs.shape[2] <= FEW_ROWS:
         return {name: fn() for name, fn in jobs.items()}
     main = torch.cuda.current_stream()
@@ -43,12 +44,10 @@ def _fan_out(jobs, inputs):
         side.wait_event(ready)
         inputs.record_stream(side)
     out = {}
-    try:
+    with K.on_streams(sides, main) as turn:
         for i, (name, fn) in enumerate(jobs.items()):
-            K._set_stream(sides[i % len(sides)])
+            turn(i)
             out[name] = fn()
-    finally:
-        K._set_stream(main)
     for side in sides:
         main.wait_stream(side)
     for t in out.values():

@@ -243,9 +243,9 @@ class RwkvLmEs:
         for side in self.streams:
             side.wait_event(ready)
             z.record_stream(side)
-        try:
+        with K.on_streams(self.streams, main) as turn:
             for i, ((l, name), key) in enumerate(self.keys.items()):
-                K._set_stream(self.streams[i % len(self.streams)])
+                turn(i)
                 W = self.blocks[l][name]
                 a, b = W.shape
                 K.es_update(z, 0, key, c.rank, c.sigma, epoch, c.noise_reuse, a, b, scale,
@@ -254,8 +254,6 @@ class RwkvLmEs:
                               self.v[(l, name)], step_t=self.step_t, beta1=c.beta1,
                               beta2=c.beta2, eps=c.eps,
                               wd=c.weight_decay if c.solver == ADAMW else 0.0)
-        finally:
-            K._set_stream(main)
         for side in self.streams:
             main.wait_stream(side)
         return z

@@ -171,12 +171,10 @@ class SpikingAttentionEs:
         sides = self._side_streams()
         for side in sides:
             side.wait_event(ready)
-        try:
+        with K.on_streams(sides, main) as turn:
             for i, fn in enumerate(calls):
-                K._set_stream(sides[i % len(sides)])
+                turn(i)
                 fn()
-        finally:
-            K._set_stream(main)
         for side in sides:
             main.wait_stream(side)
 
@@ -303,9 +301,9 @@ class SpikingAttentionEs:
         for side in self._side_streams():
             side.wait_event(ready)
             z.record_stream(side)
-        try:
+        with K.on_streams(self.streams, main) as turn:
             for i, (name, (a, b), cls) in enumerate(self.leaves):
-                K._set_stream(self.streams[i % len(self.streams)])
+                turn(i)
                 if cls == MM:
                     K.es_update(z, 0, self.keys[name], c.rank, c.sigma, epoch, c.noise_reuse, a,
                                 b, scale, out=self.grads[name])
@@ -315,8 +313,6 @@ class SpikingAttentionEs:
                 K.solver_step(c.solver, c.lr, self.P[name], self.grads[name], self.m[name],
                               self.v[name], step_t=self.step_t, beta1=c.beta1, beta2=c.beta2,
                               eps=c.eps, wd=c.weight_decay if c.solver == ADAMW else 0.0)
-        finally:
-            K._set_stream(main)
         for side in self.streams:
             main.wait_stream(side)
         return z
