@@ -432,8 +432,8 @@ __device__ __forceinline__ bool parts_whole(float v) {
 //   (x B_m) A_m^T   one k slice at the end.  Each fp32 factor is the sum of three
 //           bf16 parts (8 significant bits each), and the six products p + q <= 2
 //           fill 6 of the 8 k of a lane: half a slice per member, so the term keeps
-//           fp32 accuracy and one rounding.  A tile with a factor or an x B_m
-//           outside 2^-50 .. 2^60 (parts_whole) takes fp32 products instead.
+//           fp32 accuracy and one rounding.  An output with a factor or an x B_m
+//           outside 2^-50 .. 2^60 (parts_whole) takes their fp32 product instead.
 // F: the output-side factor rows (fp32, member pitch a + b); Fb: the input-side
 // rows as bf16 (member pitch b).
 // At 100000 x 512 -> 2048 (bf16 x and y, relu^2, 100 rows per member) the call
@@ -614,19 +614,14 @@ void k_gemm_bf16_dl(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, co
 
     // ---- (x B_m) A_m^T as one k slice per two members --------------------------------
     if constexpr (NOISY) {
-        // lane lc (hl 0) of wave (wr, wc): row 64 wr + 32 wc + lc, element m its
-        // product with member m's factor
-        const int32_t xbr = 64 * wr + 32 * wc + lc;
-        const int32_t xbm = nm == 1 || xbr >= rows_here ? 0 : tr.member(P, xbr);
-        const float xb = xbm == 0 ? xba[0] : xbm == 1 ? xba[1] : xbm == 2 ? xba[2] : xba[3];
-        bool plain = hl == 0 && xbr < rows_here && !parts_whole(xb);
-#pragma unroll
-        for (int m = 0; m < DL_NM; ++m) plain |= m < nm && !parts_whole(ao[m]);
-        // every wave is past its last read of the stages
-        plain = __syncthreads_or(plain);
+        __syncthreads();  // every wave is past its last read of the stages
         uint4* AF = reinterpret_cast<uint4*>(smem);  // [nm][256] output-side fragments
         uint4* XF = AF + DL_NM * KB_BN;              // [128] x B_m fragments
-        // products k: a0 x0, a1 x0, a0 x1, a1 x1, a2 x0, a0 x2 (plain: the fp32 factors)
+        float* AO = reinterpret_cast<float*>(XF + DL_BM);  // the operands themselves
+        float* XB = AO + DL_NM * KB_BN;
+        // products k: a0 x0, a1 x0, a0 x1, a1 x1, a2 x0, a0 x2; the parts of a value that
+        // they do not hold (parts_whole) are 0
+        uint32_t kept = 0;  // this lane's fragments hold such a value: their last word
 #pragma unroll
         for (int m = 0; m < DL_NM; ++m) {
             if (m >= nm) break;
@@ -635,16 +630,23 @@ void k_gemm_bf16_dl(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, co
             const uint32_t p1 = pack_bf16x2(r1, 0.0f);
             const uint32_t p2 = pack_bf16x2(r1 - __uint_as_float(p1 << 16), 0.0f);
             const uint32_t p01 = p0 | (p1 << 16);
-            AF[m * KB_BN + tid] = plain ? uint4{__float_as_uint(ao[m]), 0u, 0u, 0u}
-                                        : uint4{p01, p01, p2 | (p0 << 16), 0u};
+            AF[m * KB_BN + tid] = parts_whole(ao[m]) ? uint4{p01, p01, p2 | (p0 << 16), 0u}
+                                                     : uint4{0u, 0u, 0u, 1u};
+            AO[m * KB_BN + tid] = ao[m];
         }
+        // lane lc (hl 0) of wave (wr, wc): row 64 wr + 32 wc + lc, element m its
+        // product with member m's factor
+        const int32_t xbr = 64 * wr + 32 * wc + lc;
         if (hl == 0) {
-            const uint32_t p0 = pack_bf16x2(xb, 0.0f);
-            const float r1 = xb - __uint_as_float(p0 << 16);
+            const int32_t m = nm == 1 || xbr >= rows_here ? 0 : tr.member(P, xbr);
+            const float v = m == 0 ? xba[0] : m == 1 ? xba[1] : m == 2 ? xba[2] : xba[3];
+            const uint32_t p0 = pack_bf16x2(v, 0.0f);
+            const float r1 = v - __uint_as_float(p0 << 16);
             const uint32_t p1 = pack_bf16x2(r1, 0.0f);
             const uint32_t p2 = pack_bf16x2(r1 - __uint_as_float(p1 << 16), 0.0f);
-            XF[xbr] = plain ? uint4{__float_as_uint(xb), 0u, 0u, 0u}
-                            : uint4{p0 | (p0 << 16), p1 | (p1 << 16), p0 | (p2 << 16), 0u};
+            XF[xbr] = parts_whole(v) ? uint4{p0 | (p0 << 16), p1 | (p1 << 16), p0 | (p2 << 16), 0u}
+                                     : uint4{0u, 0u, 0u, 1u};
+            XB[xbr] = v;
         }
         __syncthreads();
         int32_t rm[2];
@@ -653,34 +655,41 @@ void k_gemm_bf16_dl(LinParams P, const uint16_t* __restrict__ Wb, int32_t kp, co
             const int32_t row = 64 * wr + 32 * i + lc;
             rm[i] = nm == 1 || row >= rows_here ? 0 : tr.member(P, row);
         }
-        for (int32_t t = 0; 2 * t < nm && !plain; ++t) {
+        for (int32_t t = 0; 2 * t < nm; ++t) {
             const int32_t m = 2 * t + hl;  // this lane half's member
             u16x8 xf[2];
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 uint4 v = XF[64 * wr + 32 * i + lc];
+                kept |= v.w;
+                v.w = 0u;
                 if (rm[i] != m) v = uint4{0u, 0u, 0u, 0u};
                 xf[i] = __builtin_bit_cast(u16x8, v);
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const uint4 v = AF[min(m, nm - 1) * KB_BN + 128 * wc + 32 * j + lc];
+                uint4 v = AF[min(m, nm - 1) * KB_BN + 128 * wc + 32 * j + lc];
+                kept |= v.w;
+                v.w = 0u;
                 const u16x8 af = __builtin_bit_cast(u16x8, v);
 #pragma unroll
                 for (int i = 0; i < 2; ++i) acc[i][j] = mfma32b(af, xf[i], acc[i][j]);
             }
         }
-        if (plain) {
+        if (__ballot(kept != 0) != 0) {
+            // outputs with such an operand: the fp32 product (the MFMAs added 0)
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
-                const uint4* ar = AF + rm[i] * KB_BN + 128 * wc + 4 * hl;
-                const float x = __uint_as_float(XF[64 * wr + 32 * i + lc].x);
+                const float x = XB[64 * wr + 32 * i + lc];
+                const bool xw = parts_whole(x);
+                const float* ar = AO + rm[i] * KB_BN + 128 * wc + 4 * hl;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
-                        const float a1 = __uint_as_float(ar[32 * j + 8 * (e >> 2) + (e & 3)].x);
-                        acc[i][j][e] = __fadd_rn(acc[i][j][e], __fmul_rn(x, a1));
+                        const float f = ar[32 * j + 8 * (e >> 2) + (e & 3)];
+                        const float y = __fadd_rn(acc[i][j][e], __fmul_rn(x, f));
+                        acc[i][j][e] = xw && parts_whole(f) ? acc[i][j][e] : y;
                         if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // few values live at a time
                     }
             }
