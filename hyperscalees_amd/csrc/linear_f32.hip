@@ -445,7 +445,14 @@ void k_gemm_f32s(LinParams P, const float* __restrict__ F, const uint16_t* __res
     };
     // accumulator element e of lane l: row 8 (e / 4) + 4 kh + e % 4 of the
     // 32-row tile, column lc
-    bool bad = false;
+    auto past = [](float v) {
+        const float a = fabsf(v);
+        return !(a < INFINITY) || (a < 0x1p-60f && a > 0.0f);
+    };
+    // the largest of (bits of |sum|) - (bits of 2^-60), doubled: one of a sum past either
+    // bound, or of 0, is at least that of infinity
+    constexpr uint32_t kLow = 0x21800000u << 1, kInf = 0x7f800000u << 1;
+    uint32_t far = 0;
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -458,8 +465,7 @@ void k_gemm_f32s(LinParams P, const float* __restrict__ F, const uint16_t* __res
                 const int32_t col = wn0 + 32 * j + lc;
                 if (col >= ct) continue;
                 const float yv = __fadd_rn(acc[i][j][e], low[i][j][e]);
-                const float ay = fabsf(yv);
-                bad |= !(ay < INFINITY) || (ay < 0x1p-60f && ay > 0.0f);
+                far = max(far, (__float_as_uint(yv) << 1) - kLow);
                 yrow[col] = noisy ? add_noise(yv, row, col) : yv;
             }
         }
@@ -467,21 +473,37 @@ void k_gemm_f32s(LinParams P, const float* __restrict__ F, const uint16_t* __res
     // finite and leaves its row or column of sums so.  Parts below 2^-126 lose bits
     // (operands under 2^-102, split3): b 2^-126 times the other operand, less than
     // the fp32 sums' own rounding where |y| >= 2^-60 and the operands are below 2^42.
-    // Past either bound the wave forms its outputs again with plain fp32 chains,
-    // which give what fp32 gives (sums of exactly 0, as of rows of zeros, stand).
-    if (__any(bad)) {
-#pragma unroll 1
-        for (int32_t e = lane; e < WM * WN; e += 64) {
-            const int32_t row = wm0 + e / WN, col = wn0 + e % WN;
-            if (row >= rows_here || col >= ct) continue;
+    // Outputs past either bound are formed again with plain fp32 chains, which give what
+    // fp32 gives (sums of exactly 0, as of rows of zeros, stand), each by its lane, so
+    // that rows of small values do not slow down the others (16384 x 1024 -> 1024 with
+    // one row in 128 scaled by 2^-80: 0.55 ms, and 21 with the wave's outputs; 0.26
+    // without such rows).
+    if (!__any(far >= kInf - kLow)) return;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            uint32_t left = 0;  // this lane's outputs of the 32 x 32 tile, a bit each
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int32_t row = wm0 + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
+                if (row < rows_here && past(__fadd_rn(acc[i][j][e], low[i][j][e]))) left |= 1u << e;
+            }
+            const int32_t col = wn0 + 32 * j + lc;
+            if (col >= ct) left = 0;
             const float* w = P.W + (P.tmm ? o0 + col : (int64_t)(o0 + col) * b);
-            const int64_t wk = P.tmm ? P.a : 1, xo = xoffs[row];
-            float yv = 0.0f;
+            const int64_t wk = P.tmm ? P.a : 1;
 #pragma unroll 1
-            for (int32_t k = 0; k < b; ++k) yv = __builtin_fmaf(x_at<XFMT>(P.x, xo, k), w[k * wk], yv);
-            P.y[yoffs[row] + col] = noisy ? add_noise(yv, row, col) : yv;
+            for (; left; left &= left - 1) {
+                const int32_t e = __builtin_ctz(left);
+                const int32_t row = wm0 + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
+                const int64_t xo = xoffs[row];
+                float yv = 0.0f;
+#pragma unroll 1
+                for (int32_t k = 0; k < b; ++k) yv = __builtin_fmaf(x_at<XFMT>(P.x, xo, k), w[k * wk], yv);
+                P.y[yoffs[row] + col] = noisy ? add_noise(yv, row, col) : yv;
+            }
         }
-    }
 }
 
 // ---- k_gemm_f32 ------------------------------------------------------------------

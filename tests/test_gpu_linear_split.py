@@ -122,3 +122,25 @@ def test_split_values_without_parts(hses_gpu):
     np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
     np.testing.assert_array_equal(y[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
     assert (np.abs(y[fin] - ref[fin]) <= 2.0 ** -24 * (4 * np.sqrt(inp) + 8) * s[fin]).all()
+
+
+@pytest.mark.parametrize("value", [2.0 ** -80, 0.0, np.inf])
+def test_split_rows_past_the_range_leave_others_alone(hses_gpu, value):
+    """A row of sums below 2^-60, of zeros or of infinities in a tile: the other rows keep
+    their bits (only its own outputs are formed again on fp32 chains)."""
+    rng = np.random.default_rng(5)
+    n, inp, out = 260, 130, 300
+    x = torch.from_numpy(rng.standard_normal((n, inp)).astype(np.float32)).cuda()
+    W = torch.from_numpy(rng.standard_normal((out, inp)).astype(np.float32)).cuda()
+
+    def run():
+        return hses_gpu.perturbed_linear(x.view(1, n, inp), W, KEY, 1, 0.2, 0, 0, 0, n // 4, 4).view(n, out)
+
+    before = run().clone()
+    rows = torch.tensor([0, 77, 259], device="cuda")
+    x[rows] = x[rows].sign() * value if value < np.inf else value
+    after = run()
+    keep = torch.ones(n, dtype=torch.bool, device="cuda")
+    keep[rows] = False
+    assert torch.equal(after[keep], before[keep])
+    assert not torch.equal(after[rows], before[rows])
