@@ -136,9 +136,12 @@ __global__ __launch_bounds__(256) void k_sa_encode(const float* __restrict__ cq,
 // mask, so a step needs no reduction over lanes.  Head sizes 8, 16 and 32 have their own
 // instances: a lane's key (hd values) and its V column (64) stay in registers over
 // its wave's rows, and only the uniform q and the p rows are read from LDS, four at a
-// time.  Other sizes read K and V from LDS.
-// 1024 members x 4 heads, 64 tokens, head size 16, 8 steps: 138 -> 94 us (a reduction over
-// lanes in every step, K and V from LDS in every group).
+// time.  Other sizes read K and V from LDS: no configuration here has them, and an
+// instance of 64 would hold 128 values a lane.
+// Calls of 1024 members x 4 heads, 64 tokens, 8 steps, against a reduction over lanes in
+// every step and K and V from LDS in every group: head size 8 121 -> 71 us, 16 125 -> 85,
+// 32 259 -> 107; the general form 4 113 -> 78, 48 660 -> 352, 64 922 -> 503 (17 tokens: 4
+// 35 -> 23, 64 147 -> 49).
 constexpr int kSaWaves = 4;
 constexpr int kSaMaxR = 64, kSaMaxHd = 64;
 constexpr int kSaPP = kSaMaxR + 4;  // pitch of a wave's p rows (16-byte reads, distinct banks)

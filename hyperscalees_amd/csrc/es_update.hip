@@ -23,7 +23,8 @@
 //     barrier per chunk).  hses_es_update_rec runs the same kernel on the
 //     forward's factor record, so the two agree bit for bit.
 // Without a workspace for the record (hses_es_update_noalloc's fixed scratch, a
-// caller's workspace that holds the partials alone, or r >= 32 with a split's record past the bound) the contraction draws:
+// caller's workspace that holds the partials alone, or r >= 32 with a split's record
+// past the bound) the contraction draws:
 //   k_es_partial (r < 32): 128x128 tiles, fp32 MFMA, a k-chunk of 32 columns holds
 //     32 / r pairs, so every thread generates a run of stream rows per chunk.
 //   k_es_rows<.., false>: the generation of the next rank chunk is interleaved with
@@ -492,7 +493,9 @@ __global__ __launch_bounds__(R_MAXT) void k_es_rows(UpdParams P, RowTiles G) {
 // pair after one jump.  WEIGHT (k_es_gemm): the A rows (stream rows b ..) are
 // stored as (v * bs) * w with the pair's weight w, the reference's fp32 products,
 // and the last block writes k_es_gemm's fp32 flag to scale[0].  Bound by the draw's
-// vector instructions (106 per normal, 300 G normals/s).
+// vector instructions (106 per normal) and, at small ranks, the threads' jumps: 275 G
+// normals/s for 1501 pairs x 700 rows at rank 48 (48 normals a thread and jump), 156 for
+// 2048 pairs x 2048 rows at rank 1 (16).
 template <bool WEIGHT>
 __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int32_t pairs, int32_t groups,
                                                  float* __restrict__ rec, int32_t vec,
@@ -567,7 +570,7 @@ __global__ __launch_bounds__(256) void k_es_draw(UpdParams P, int32_t pair0, int
 // rows, one chunk ahead.  48 KB of LDS (64-byte rows per part, pieces swizzled by
 // slot_of) and two waves per SIMD let two workgroups share a CU, one's conversion and
 // barriers beside the other's MFMAs.  1024 x 1024 at rank 1 and 4096 members (K 2048,
-// 8 splits of 8 chunks): 40 us of the call's 69 (draw 27, reduction 11), against 202 us
+// 8 splits of 8 chunks): 41 us of the call's 70 (draw 27, reduction 11), against 202 us
 // drawing in the contraction.  On fp16 high and low parts and three products (22 bits)
 // it took 30, but the error was up to 2.4 times that of fp32 operands at few members
 // and 1.2 times at many; with the bf16 parts it is 0.3 to 1.0 of it (1 to 4096

@@ -512,8 +512,9 @@ void k_gemm_f32s(LinParams P, const float* __restrict__ F, const uint16_t* __res
 // eight: 70% of the kernel's LDS cycles at 16 -> 64, rank 8), reads them once when
 // the tile has one member, and takes each row's offset and member from an LDS
 // table (the divisions of 16 rows per lane were most of its vector instructions).
-// Bits do not change: 524288 x 16 -> 64 at rank 8 166 -> 121 us (best 78), 32768 spike
-// rows 256 -> 256 at rank 4 83 -> 65 us.
+// Bits do not change.  Whole calls: 524288 x 16 -> 64 at rank 8 168 -> 83 us, spike rows at
+// rank 4 131072 x 128 -> 128 84 -> 73 and 131072 x 784 -> 128 316 -> 305 (its MFMAs bound
+// it), 32768 spike rows 200 -> 200 at rank 8 and 16 rows a member 89 -> 64.
 //
 // NT 32-column MFMA tiles per wave (BN = 32 NT); four waves of 32 rows.  RK is
 // the rank padded to 1, 4, 8 or 16 (the LDS copies of B_m and A_m rows hold RK

@@ -217,6 +217,10 @@ int hses_lif_scan(const float *d_cur, const float *d_v0, int32_t T, int64_t rows
  * and, for large ranks, one per-workgroup staging slot for a pair's B factor;
  * the (n, b, r) factor tensor itself is never materialised).  Large ranks
  * (r a multiple of 16, r <= 128, a <= 128) need math = HSES_MATH_BF16.  With
+ * math = HSES_MATH_F32, outputs at least 256 wide over more than 64 inputs (and do_Tmm)
+ * take every fp32 operand of x W^T as three bf16 parts (its 24 bits; six part products,
+ * bf16 x and spikes three) and outputs below 2^-60 or not finite as fp32 chains; x B_m
+ * and (x B_m) A_m^T are fp32 throughout.  With
  * math = HSES_MATH_BF16 and small ranks (members per 128-row tile x rank <= 16)
  * the wide-output kernel runs when the workspace holds its bf16 copy of W and x
  * rows are 16-byte aligned; otherwise the small-rank kernel (no workspace). */
