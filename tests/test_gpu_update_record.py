@@ -47,7 +47,7 @@ def test_own_record(hses_gpu, a, b, r, n, tid_lo):
 
 def test_zero_fitness_and_scale_range(hses_gpu):
     """All-zero fitness gives zeros; fitness at either end of fp32 keeps the
-    relative bar (the operand scale follows max |f|)."""
+    relative bar (the operands keep fp32's range)."""
     fit = np.zeros(64, np.float32)
     assert not gpu_grad(hses_gpu, 0.1, 2, fit, 40, 50, np.float32(1.0)).any()
     base = np.random.default_rng(1).standard_normal(64).astype(np.float32)
